@@ -100,7 +100,25 @@ class TQRowsAppendArgs(ctypes.Structure):
     ]
 
 
+class TQStoreArgs(ctypes.Structure):
+    """anna_mi_tq_store_args."""
+
+    _fields_ = [
+        ("dtype", _I), ("key_format", _I), ("batch", _I64), ("row0", _I64), ("rows", _I64), ("kv_heads", _I64),
+        ("head_dim", _I64), ("tokens", _I64), ("capacity", _I64), ("residual_capacity", _I64), ("key_bits", _I),
+        ("value_bits", _I), ("value_group_size", _I64), ("new_key", _P), ("new_value", _P),
+        ("key_stride_row", _I64), ("key_stride_head", _I64), ("key_stride_token", _I64),
+        ("value_stride_row", _I64), ("value_stride_head", _I64), ("value_stride_token", _I64),
+        ("key_codes", _P), ("key_norms", _P), ("key_signs", _P), ("key_residual_norms", _P), ("key_dense", _P),
+        ("value_data", _P), ("value_scales", _P), ("value_zeros", _P), ("residual_key", _P), ("residual_value", _P),
+        ("seq_in", _P), ("seq_out", _P), ("past_out", _P), ("max_leaving", _I64), ("max_fill", _I64),
+        ("signs", _P), ("thresholds", _P), ("centroids", _P), ("gaussian", _P), ("gaussian_t", _P),
+        ("value_lane_groups", _I), ("k0", _F),
+    ]
+
+
 PROTOTYPES.update({
+    "anna_mi_tq_store": [ctypes.POINTER(TQStoreArgs), _P],
     "anna_mi_tq_rows_append": [ctypes.POINTER(TQRowsAppendArgs), _P],
     "anna_mi_tq_pack_kv": [ctypes.POINTER(TQPackArgs), _P],
     "anna_mi_tq_decode": [ctypes.POINTER(TQDecodeArgs), _P],
@@ -166,6 +184,7 @@ RAW_PROTOTYPES: dict[str, tuple] = {
     "anna_mi_sizeof_tq_append_args": (_I64, []),
     "anna_mi_sizeof_tq_pack_args": (_I64, []),
     "anna_mi_sizeof_tq_rows_append_args": (_I64, []),
+    "anna_mi_sizeof_tq_store_args": (_I64, []),
     "anna_mi_tq_decode_workgroups": (_I64, [_I64, _I64, _P, _I64]),
 }
 

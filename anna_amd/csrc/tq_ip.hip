@@ -26,11 +26,10 @@
 
 #include "common.hpp"
 #include "tq_hadamard.hpp"
+#include "tq_ip_core.hpp"
 
 namespace anna {
 namespace {
-
-constexpr int IPNV = 4;  // vectors per wave
 
 // out[n][e] (index lane*E + e) = sum_k M[k*D + lane*E + e] * vl[n*D + k], k ascending (one fma
 // chain from 0).  vl: the wave's vectors in LDS.
@@ -65,135 +64,89 @@ __device__ __forceinline__ void matvec_wave_n(const float* __restrict__ M, const
   }
 }
 
-// y = fl(1/sqrt(D)) * FWHT(s .* x), as the TQ-MSE quantizer forms it
-template <int NV, int E>
-__device__ __forceinline__ void rotate_wave_n(const float (&x)[NV][E], const float* __restrict__ signs, float inv,
-                                              float (&y)[NV][E]) {
-  const int lane = threadIdx.x & 63;
-  float sg[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) sg[e] = signs[lane * E + e];
-#pragma unroll
-  for (int n = 0; n < NV; ++n)
-#pragma unroll
-    for (int e = 0; e < E; ++e) y[n][e] = x[n][e] * sg[e];
-  fwht_wave_n<NV, E>(y);
-#pragma unroll
-  for (int n = 0; n < NV; ++n)
-#pragma unroll
-    for (int e = 0; e < E; ++e) y[n][e] = y[n][e] * inv;
-}
-
-// 4 waves per 256-thread workgroup, IPNV vectors per wave, lane l holds elements l*E .. l*E+E-1.
-// Every wave reaches the barrier (a wave past the end works on clamped copies and stores nothing).
-template <int XDT, int E>
-__global__ __launch_bounds__(256) void tq_ip_quantize_kernel(
-    const typename Elem<XDT>::T* __restrict__ x, int64_t nvec, int64_t D, int64_t xs,
-    const float* __restrict__ signs, const float* __restrict__ thr, const float* __restrict__ cent, int nthr,
-    const float* __restrict__ gt, uint8_t* __restrict__ idx_out, uint8_t* __restrict__ qjl_out,
-    float* __restrict__ norm_out, float* __restrict__ rn_out) {
-  __shared__ float rl[4][IPNV * 64 * E];
+// Tiles of TV vectors per 512-thread workgroup (the D x D products on the matrix cores,
+// tq_ip_core.hpp), TV / 8 per wave, lane l holding elements l*E .. l*E+E-1.  Every wave reaches the
+// barriers (one past the end works on clamped copies and stores nothing).  Bound by the fp32 matrix
+// rate (2 D^2 flops per vector and kernel); one wave per 4 vectors with scalar fma re-read the
+// matrix from L2 for each wave.
+template <int XDT, int E, int TV>
+__global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_quantize_kernel(
+    const typename Elem<XDT>::T* __restrict__ x, int64_t nvec, int64_t xs, const float* __restrict__ signs,
+    const float* __restrict__ thr, const float* __restrict__ cent, int nthr, const float* __restrict__ gt,
+    uint8_t* __restrict__ idx_out, uint8_t* __restrict__ qjl_out, float* __restrict__ norm_out,
+    float* __restrict__ rn_out) {
+  extern __shared__ __attribute__((aligned(16))) float ip_lds[];
+  constexpr int D = 64 * E, VW = TV / IP_WAVES, NB = VW < 4 ? VW : 4;
   const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * IPNV;
-  float xv[IPNV][E];
+  const int64_t v0 = (int64_t)blockIdx.x * TV + wave * VW;
 #pragma unroll
-  for (int n = 0; n < IPNV; ++n) {
-    int64_t v = v0 + n < nvec ? v0 + n : nvec - 1;
+  for (int n0 = 0; n0 < VW; n0 += NB) {
+    float xv[NB][E], rho[NB][E], nrm[NB], rn[NB];
+    uint32_t code[NB][E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) xv[n][e] = Elem<XDT>::load(x, v * xs + lane * E + e);
-  }
-  float ss[IPNV], nrm[IPNV];
-  sumsq_wave_n<IPNV, E>(xv, ss);
+    for (int n = 0; n < NB; ++n) {
+      const int64_t v = v0 + n0 + n < nvec ? v0 + n0 + n : nvec - 1;
 #pragma unroll
-  for (int n = 0; n < IPNV; ++n) nrm[n] = __builtin_sqrtf(ss[n]);
-  float y[IPNV][E];
-  rotate_wave_n<IPNV, E>(xv, signs, tq_inv_sqrt(D), y);
-  uint32_t code[IPNV][E];
-  float rho[IPNV][E];
-#pragma unroll
-  for (int n = 0; n < IPNV; ++n)
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      uint32_t c = 0;
-      for (int j = 0; j < nthr; ++j) c += y[n][e] >= __fmul_rn(thr[j], nrm[n]) ? 1u : 0u;
-      code[n][e] = c;
-      rho[n][e] = __builtin_fmaf(-cent[c], nrm[n], y[n][e]);
+      for (int e = 0; e < E; ++e) xv[n][e] = Elem<XDT>::load(x, v * xs + lane * E + e);
     }
-  float gg[IPNV];
-  sumsq_wave_n<IPNV, E>(rho, gg);
-  float* my = rl[wave];
+    ip_mse_stage<NB, E>(xv, signs, thr, cent, nthr, code, nrm, rho, rn);
 #pragma unroll
-  for (int n = 0; n < IPNV; ++n)
+    for (int n = 0; n < NB; ++n) {
+      const int64_t v = v0 + n0 + n;
+      float* my = ip_lds + (wave * VW + n0 + n) * IP_ROW<E>;
 #pragma unroll
-    for (int e = 0; e < E; ++e) my[n * D + lane * E + e] = rho[n][e];
-  __syncthreads();
-  float z[IPNV][E];
-  matvec_wave_n<IPNV, E>(gt, my, D, z);
+      for (int e = 0; e < E; ++e) my[ip_pos(lane * E + e)] = rho[n][e];
+      if (v >= nvec) continue;
 #pragma unroll
-  for (int n = 0; n < IPNV; ++n) {
+      for (int e = 0; e < E; ++e) idx_out[v * D + lane * E + e] = (uint8_t)code[n][e];
+      if (lane == 0) {
+        norm_out[v] = nrm[n];
+        rn_out[v] = rn[n];
+      }
+    }
+  }
+  ip_signs<E, TV>(gt, ip_lds, wave);
+#pragma unroll
+  for (int n = 0; n < VW; ++n) {
     const int64_t v = v0 + n;
     if (v >= nvec) break;
-    uint8_t* ib = idx_out + v * D + lane * E;
-    uint8_t* qb = qjl_out + v * D + lane * E;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      ib[e] = (uint8_t)code[n][e];
-      qb[e] = z[n][e] >= 0.f ? 1 : 0;
-    }
-    if (lane == 0) {
-      norm_out[v] = nrm[n];
-      rn_out[v] = nrm[n] > 0.f ? __fdiv_rn(__builtin_sqrtf(gg[n]), nrm[n]) : 0.f;
-    }
+    for (int e = 0; e < E; ++e)
+      qjl_out[v * D + lane * E + e] = ip_lds[(wave * VW + n) * IP_ROW<E> + ip_pos(lane * E + e)] > 0.f ? 1 : 0;
   }
 }
 
-template <int ODT, int E>
-__global__ __launch_bounds__(256) void tq_ip_dequant_kernel(
+template <int ODT, int E, int TV>
+__global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_dequant_kernel(
     const uint8_t* __restrict__ idx, const uint8_t* __restrict__ qjl, const float* __restrict__ norms,
-    const float* __restrict__ rn, int64_t nvec, int64_t D, const float* __restrict__ signs,
-    const float* __restrict__ cent, const float* __restrict__ g, float k0, typename Elem<ODT>::T* __restrict__ out,
-    int64_t os) {
-  __shared__ float sl[4][IPNV * 64 * E];
+    const float* __restrict__ rn, int64_t nvec, const float* __restrict__ signs, const float* __restrict__ cent,
+    const float* __restrict__ g, float k0, typename Elem<ODT>::T* __restrict__ out, int64_t os) {
+  extern __shared__ __attribute__((aligned(16))) float ip_lds[];
+  constexpr int D = 64 * E, VW = TV / IP_WAVES;
   const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int64_t v0 = ((int64_t)blockIdx.x * 4 + wave) * IPNV;
-  float* my = sl[wave];
-  float c[IPNV][E];
+  const int64_t v0 = (int64_t)blockIdx.x * TV + wave * VW;
 #pragma unroll
-  for (int n = 0; n < IPNV; ++n) {
+  for (int n = 0; n < VW; ++n) {
     const int64_t v = v0 + n < nvec ? v0 + n : nvec - 1;
+    float* my = ip_lds + (wave * VW + n) * IP_ROW<E>;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      c[n][e] = cent[idx[v * D + lane * E + e]];
-      my[n * D + lane * E + e] = qjl[v * D + lane * E + e] ? 1.f : -1.f;
-    }
+    for (int e = 0; e < E; ++e) my[ip_pos(lane * E + e)] = qjl[v * D + lane * E + e] ? 1.f : -1.f;
   }
   __syncthreads();
-  float w[IPNV][E];
-  matvec_wave_n<IPNV, E>(g, my, D, w);
-  const float inv = tq_inv_sqrt(D);
+  ip_project<E, TV>(g, ip_lds, wave);
   float sg[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) sg[e] = signs[lane * E + e];
-  float nrm[IPNV];
 #pragma unroll
-  for (int n = 0; n < IPNV; ++n) {
-    const int64_t v = v0 + n < nvec ? v0 + n : nvec - 1;
-    const float coef = k0 * rn[v];
-    nrm[n] = norms[v];
-#pragma unroll
-    for (int e = 0; e < E; ++e) w[n][e] = __builtin_fmaf(coef, w[n][e], c[n][e]);
-  }
-  fwht_wave_n<IPNV, E>(w);
-#pragma unroll
-  for (int n = 0; n < IPNV; ++n) {
+  for (int n = 0; n < VW; ++n) {
     const int64_t v = v0 + n;
     if (v >= nvec) break;
+    float c[E], o[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      float t = w[n][e] * inv;
-      t = t * sg[e];
-      out[v * os + lane * E + e] = Elem<ODT>::cvt(nrm[n] * t);
-    }
+    for (int e = 0; e < E; ++e) c[e] = cent[idx[v * D + lane * E + e]];
+    ip_reconstruct<E>(ip_lds + (wave * VW + n) * IP_ROW<E>, c, k0 * rn[v], norms[v], sg, lane, o);
+#pragma unroll
+    for (int e = 0; e < E; ++e) out[v * os + lane * E + e] = Elem<ODT>::cvt(o[e]);
   }
 }
 
@@ -304,7 +257,15 @@ void dispatch_e(int64_t D, F&& go) {
 
 bool ip_dim_ok(int64_t D) { return D == 64 || D == 128 || D == 256 || D == 512 || D == 1024; }
 
-float ip_k0(int64_t D) { return (float)(1.2533141373155002512 / (double)D); }
+// Tiles of 16 while that leaves at most 32 vectors per compute unit, else the large tile.
+bool ip_small(int64_t nvec) { return nvec < 256 * 32; }
+
+template <class K>
+int ip_raise_lds(K kern, size_t lds, const char* what) {
+  ANNA_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess,
+             "%s: cannot raise the LDS limit", what);
+  return ANNA_MI_OK;
+}
 
 }  // namespace
 }  // namespace anna
@@ -331,16 +292,26 @@ extern "C" int anna_mi_tq_ip_quantize(const void* x, int x_dtype, int64_t nvec, 
   ANNA_CHECK(ip_dim_ok(D), "anna_mi_tq_ip_quantize: head_dim must be a power of two in [64, 1024]");
   ANNA_CHECK(x_row_stride >= D, "anna_mi_tq_ip_quantize: row stride smaller than head_dim");
   ANNA_CHECK(nvec > 0, "anna_mi_tq_ip_quantize: negative vector count");
-  const dim3 grid((unsigned)((nvec + 4 * IPNV - 1) / (4 * IPNV)));
   const int nthr = (1 << (bits - 1)) - 1;
+  int rc = ANNA_MI_OK;
   ANNA_DISPATCH_DTYPE(x_dtype, XDT, {
     dispatch_e(D, [&](auto e_tag) {
       constexpr int E = decltype(e_tag)::value;
-      hipLaunchKernelGGL((tq_ip_quantize_kernel<XDT, E>), grid, dim3(256), 0, as_stream(stream),
-                         (const typename Elem<XDT>::T*)x, nvec, D, x_row_stride, signs, thresholds, centroids, nthr,
-                         gaussian_t, mse_indices, qjl_signs, norms, residual_norms);
+      auto go = [&](auto tv_tag) {
+        constexpr int TV = decltype(tv_tag)::value;
+        auto kern = tq_ip_quantize_kernel<XDT, E, TV>;
+        constexpr size_t lds = ip_lds_bytes<E>(TV);
+        rc = ip_raise_lds(kern, lds, "anna_mi_tq_ip_quantize");
+        if (rc != ANNA_MI_OK) return;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((nvec + TV - 1) / TV)), dim3(64 * IP_WAVES), lds, as_stream(stream),
+                           (const typename Elem<XDT>::T*)x, nvec, x_row_stride, signs, thresholds, centroids, nthr,
+                           gaussian_t, mse_indices, qjl_signs, norms, residual_norms);
+      };
+      if (ip_small(nvec)) go(std::integral_constant<int, ip_tile(E, true)>{});
+      else go(std::integral_constant<int, ip_tile(E, false)>{});
     });
   });
+  if (rc != ANNA_MI_OK) return rc;
   ANNA_LAUNCH_CHECK("tq_ip_quantize_kernel");
   return ANNA_MI_OK;
 }
@@ -357,15 +328,25 @@ extern "C" int anna_mi_tq_ip_dequant(const uint8_t* mse_indices, const uint8_t* 
   ANNA_CHECK(ip_dim_ok(D), "anna_mi_tq_ip_dequant: head_dim must be a power of two in [64, 1024]");
   ANNA_CHECK(out_row_stride >= D, "anna_mi_tq_ip_dequant: row stride smaller than head_dim");
   ANNA_CHECK(nvec > 0, "anna_mi_tq_ip_dequant: negative vector count");
-  const dim3 grid((unsigned)((nvec + 4 * IPNV - 1) / (4 * IPNV)));
+  int rc = ANNA_MI_OK;
   ANNA_DISPATCH_DTYPE(out_dtype, ODT, {
     dispatch_e(D, [&](auto e_tag) {
       constexpr int E = decltype(e_tag)::value;
-      hipLaunchKernelGGL((tq_ip_dequant_kernel<ODT, E>), grid, dim3(256), 0, as_stream(stream), mse_indices, qjl_signs,
-                         norms, residual_norms, nvec, D, signs, centroids, gaussian, ip_k0(D),
-                         (typename Elem<ODT>::T*)out, out_row_stride);
+      auto go = [&](auto tv_tag) {
+        constexpr int TV = decltype(tv_tag)::value;
+        auto kern = tq_ip_dequant_kernel<ODT, E, TV>;
+        constexpr size_t lds = ip_lds_bytes<E>(TV);
+        rc = ip_raise_lds(kern, lds, "anna_mi_tq_ip_dequant");
+        if (rc != ANNA_MI_OK) return;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((nvec + TV - 1) / TV)), dim3(64 * IP_WAVES), lds, as_stream(stream),
+                           mse_indices, qjl_signs, norms, residual_norms, nvec, signs, centroids, gaussian, ip_k0(D),
+                           (typename Elem<ODT>::T*)out, out_row_stride);
+      };
+      if (ip_small(nvec)) go(std::integral_constant<int, ip_tile(E, true)>{});
+      else go(std::integral_constant<int, ip_tile(E, false)>{});
     });
   });
+  if (rc != ANNA_MI_OK) return rc;
   ANNA_LAUNCH_CHECK("tq_ip_dequant_kernel");
   return ANNA_MI_OK;
 }

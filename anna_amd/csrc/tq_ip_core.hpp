@@ -1,0 +1,223 @@
+// Building blocks of the TurboQuant inner-product quantizer (definition and arithmetic order in
+// tq_ip.hip), shared by the quantizers on flat vectors and by the cache writer.
+//
+// The two D x D products of a tile of TV vectors (rho . G^T for the signs, signs . G for the
+// reconstruction) run on the fp32 matrix instruction: v_mfma_f32_16x16x4_f32 adds its four k as
+// one fma chain in ascending k from the accumulator, subnormals and overflow included (compared
+// bit by bit with the scalar chain on this chip), so the order the oracle fixes is kept while the
+// matrix is read once per 16 to 64 vectors instead of once per 4, and at twice the rate that
+// scalar fp32 fma issues at (154 TFLOP/s against 77).
+#pragma once
+
+#include "common.hpp"
+#include "tq_hadamard.hpp"
+
+namespace anna {
+
+constexpr int IP_WAVES = 8;  // waves of a workgroup of the tile kernels
+
+// Vectors of a tile: as many as keep a wave's share of the tile's outputs (TV * D / 512) within 32
+// registers; `small` for calls of few vectors, where tiles are what fills the chip.
+constexpr int ip_tile(int E, bool small) { return small || E >= 16 ? 16 : E >= 8 ? 32 : 64; }
+// LDS row of a tile: 4 floats of padding put the 16 rows x 4 chunks of an operand read on distinct banks
+template <int E> constexpr int IP_ROW = 64 * E + 4;
+template <int E> constexpr size_t ip_lds_bytes(int TV) { return (size_t)TV * IP_ROW<E> * 4; }
+
+// Position of k in a row of the product's left operand: the four k of one instruction go to the
+// four 16-lane groups, so groups of 16 k are transposed and one 16-byte read feeds four of them.
+__device__ __forceinline__ int ip_pos(int k) { return (k & ~15) | ((k & 3) << 2) | ((k >> 2) & 3); }
+
+// y = fl(1/sqrt(D)) * FWHT(s .* x), as the TQ-MSE quantizer forms it
+template <int NV, int E>
+__device__ __forceinline__ void rotate_wave_n(const float (&x)[NV][E], const float* __restrict__ signs, float inv,
+                                              float (&y)[NV][E]) {
+  const int lane = threadIdx.x & 63;
+  float sg[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) sg[e] = signs[lane * E + e];
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int e = 0; e < E; ++e) y[n][e] = x[n][e] * sg[e];
+  fwht_wave_n<NV, E>(y);
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int e = 0; e < E; ++e) y[n][e] = y[n][e] * inv;
+}
+
+// MSE stage of NV vectors of the wave (lane's E elements each): codes, norms, the rotated residual
+// and residual_norm = |rho| / norm.
+template <int NV, int E>
+__device__ __forceinline__ void ip_mse_stage(const float (&x)[NV][E], const float* __restrict__ signs,
+                                             const float* __restrict__ thr, const float* __restrict__ cent, int nthr,
+                                             uint32_t (&code)[NV][E], float (&nrm)[NV], float (&rho)[NV][E],
+                                             float (&rn)[NV]) {
+  float ss[NV];
+  sumsq_wave_n<NV, E>(x, ss);
+#pragma unroll
+  for (int n = 0; n < NV; ++n) nrm[n] = __builtin_sqrtf(ss[n]);
+  float y[NV][E];
+  rotate_wave_n<NV, E>(x, signs, tq_inv_sqrt(64 * E), y);
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      uint32_t c = 0;
+      for (int j = 0; j < nthr; ++j) c += y[n][e] >= __fmul_rn(thr[j], nrm[n]) ? 1u : 0u;
+      code[n][e] = c;
+      rho[n][e] = __builtin_fmaf(-cent[c], nrm[n], y[n][e]);
+    }
+  float gg[NV];
+  sumsq_wave_n<NV, E>(rho, gg);
+#pragma unroll
+  for (int n = 0; n < NV; ++n) rn[n] = nrm[n] > 0.f ? __fdiv_rn(__builtin_sqrtf(gg[n]), nrm[n]) : 0.f;
+}
+
+// The E bytes of a lane (elements lane * E ..) at dst + lane * E, dst 64 * E-byte rows
+template <int E>
+__device__ __forceinline__ void store_bytes_wave(const uint32_t (&v)[E], uint8_t* dst, int lane) {
+  if constexpr (E == 1) {
+    dst[lane] = (uint8_t)v[0];
+  } else if constexpr (E == 2) {
+    ((uint16_t*)dst)[lane] = (uint16_t)(v[0] | (v[1] << 8));
+  } else {
+#pragma unroll
+    for (int e = 0; e < E; e += 4)
+      ((uint32_t*)dst)[lane * (E / 4) + e / 4] = v[e] | (v[e + 1] << 8) | (v[e + 2] << 16) | (v[e + 3] << 24);
+  }
+}
+
+// A wave's column tiles of the product: tile = wave * CT + c of the D / 16 (with D = 64 only the
+// first four waves have one)
+template <int E> constexpr int IP_CT = E >= 2 ? E / 2 : 1;
+template <int E>
+__device__ __forceinline__ bool ip_has_tile(int wave) { return E >= 2 || wave < 4; }
+
+// acc[c][n]: rows 16 n .. of `lds` (ip_pos order) times M (row-major D x D, k = row), column tile c
+// of this wave, each element one fma chain over k ascending from 0.  C layout: column lane & 15,
+// rows 4 (lane >> 4) + e.
+template <int E, int NT>
+__device__ __forceinline__ void ip_product(const float* __restrict__ M, const float* lds, int wave,
+                                           f32x4 (&acc)[IP_CT<E>][NT]) {
+  constexpr int D = 64 * E, CT = IP_CT<E>;
+  // chains in flight: NT per column tile; two column tiles together where NT alone is too few to
+  // cover the instruction's latency
+  constexpr int CG = NT >= 2 || CT < 2 ? 1 : 2;
+  constexpr int KU = 32;  // k per step: the next step's matrix elements are in flight during this one
+  const int lane = threadIdx.x & 63, r = lane & 15, kq = lane >> 4;
+  const float* arow = lds + r * IP_ROW<E> + 4 * kq;
+#pragma unroll
+  for (int c0 = 0; c0 < CT; c0 += CG) {
+    const float* bcol = M + (int64_t)kq * D + (wave * CT + c0) * 16 + r;
+    float b[CG][KU / 4], bn[CG][KU / 4];
+#pragma unroll
+    for (int c = 0; c < CG; ++c) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[c0 + c][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KU / 4; ++s) b[c][s] = bcol[c * 16 + (int64_t)(4 * s) * D];
+    }
+#pragma unroll 1
+    for (int k0 = 0; k0 < D; k0 += KU) {
+      const int kn = k0 + KU < D ? k0 + KU : k0;  // (the last step reloads itself)
+#pragma unroll
+      for (int c = 0; c < CG; ++c)
+#pragma unroll
+        for (int s = 0; s < KU / 4; ++s) bn[c][s] = bcol[c * 16 + (int64_t)(kn + 4 * s) * D];
+#pragma unroll
+      for (int kk = 0; kk < KU; kk += 16) {
+        f32x4 a[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) a[n] = *(const f32x4*)(arow + n * 16 * IP_ROW<E> + k0 + kk);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int c = 0; c < CG; ++c)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+              acc[c0 + c][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n][s], b[c][kk / 4 + s], acc[c0 + c][n], 0, 0, 0);
+      }
+#pragma unroll
+      for (int c = 0; c < CG; ++c)
+#pragma unroll
+        for (int s = 0; s < KU / 4; ++s) b[c][s] = bn[c][s];
+    }
+  }
+}
+
+// Signs stage of a tile: `lds` holds rho of TV vectors (ip_pos order, every wave's rows written, no
+// barrier yet); leaves +-1 (z >= 0) there in the same order, after a barrier.
+template <int E, int TV>
+__device__ __forceinline__ void ip_signs(const float* __restrict__ gt, float* lds, int wave) {
+  constexpr int NT = TV / 16, CT = IP_CT<E>;
+  const int lane = threadIdx.x & 63, r = lane & 15, kq = lane >> 4;
+  uint32_t pos[CT][NT];  // bit e: element e of the C fragment is >= 0
+  __syncthreads();
+  if (ip_has_tile<E>(wave)) {
+    f32x4 acc[CT][NT];
+    ip_product<E, NT>(gt, lds, wave, acc);
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        pos[c][n] = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pos[c][n] |= acc[c][n][e] >= 0.f ? 1u << e : 0u;
+      }
+  }
+  __syncthreads();  // every read of rho is done
+  if (ip_has_tile<E>(wave)) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int col = ip_pos((wave * CT + c) * 16 + r);
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          lds[(16 * n + 4 * kq + e) * IP_ROW<E> + col] = (pos[c][n] >> e) & 1u ? 1.f : -1.f;
+    }
+  }
+  __syncthreads();
+}
+
+// Projection stage: `lds` holds the +-1 signs of TV vectors (ip_pos order, after a barrier); leaves
+// w = signs . G there in plain order, after a barrier.
+template <int E, int TV>
+__device__ __forceinline__ void ip_project(const float* __restrict__ g, float* lds, int wave) {
+  constexpr int NT = TV / 16, CT = IP_CT<E>;
+  const int lane = threadIdx.x & 63, r = lane & 15, kq = lane >> 4;
+  f32x4 acc[CT][NT];
+  if (ip_has_tile<E>(wave)) ip_product<E, NT>(g, lds, wave, acc);
+  __syncthreads();  // every read of the signs is done
+  if (ip_has_tile<E>(wave)) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lds[(16 * n + 4 * kq + e) * IP_ROW<E> + (wave * CT + c) * 16 + r] = acc[c][n][e];
+  }
+  __syncthreads();
+}
+
+// Reconstruction of one vector from its w row: lane's E elements of norm * R^T(c + k0 rn w).
+template <int E>
+__device__ __forceinline__ void ip_reconstruct(const float* wrow, const float (&c)[E], float coef, float nrm,
+                                               const float (&sg)[E], int lane, float (&out)[E]) {
+  float u[1][E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) u[0][e] = __builtin_fmaf(coef, wrow[lane * E + e], c[e]);
+  fwht_wave_n<1, E>(u);
+  const float inv = tq_inv_sqrt(64 * E);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    float t = u[0][e] * inv;
+    t = t * sg[e];
+    out[e] = nrm * t;
+  }
+}
+
+inline float ip_k0(int64_t D) { return (float)(1.2533141373155002512 / (double)D); }  // fl(sqrt(pi/2) / D)
+
+}  // namespace anna

@@ -597,6 +597,18 @@ def tq_ip_scores(query, idx, norms, qjl, rn, signs, centroids, gaussian_t, bits,
     return out
 
 
+def tq_store_rows(tensor):
+    """`tensor` [rows, heads, tokens, D] as anna_mi_tq_store reads it: contiguous vectors, every one
+    16-byte aligned (a copy where they are not)."""
+    per = 16 // tensor.element_size()
+    s0, s1, s2, s3 = tensor.stride()
+    if s3 != 1 or s0 % per or s1 % per or s2 % per or tensor.data_ptr() % 16:
+        tensor = tensor.contiguous()
+        if tensor.data_ptr() % 16:
+            tensor = tensor.clone()
+    return tensor
+
+
 # ---------------------------------------------------------------- tiled int4 GEMV, LM-head top-k
 # (sycl:3272-3343 xpu_int4_gemv_tiled, sycl:2137-2572 lm_head_int4_topk_fused)
 

@@ -295,20 +295,37 @@ class TurboQuantRowsCache(TurboQuantBatchCache):
             raise ValueError(f"sequence {b}: {q} quantized tokens exceed its capacity {self.capacities[b]}")
         if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
             raise ValueError("keys/values must be bf16")
-        if q > 0:
-            codes, norms = self.qn.quantize(keys[:, :q].reshape(-1, D))
-            self.key_codes[b, :, :q] = codes.view(h, q, -1)
-            self.key_norms[b, :, :q] = norms.view(h, q)
-            data, sc, zr = fused_ops.tq_values_quantize(values[:, :q], self.bits, self.value_group_size)
-            self.value_data[b, :, :q] = data
-            self.value_scales[b, :, :q] = sc
-            self.value_zeros[b, :, :q] = zr
-        if L > q:
-            slots = torch.arange(q, L, device=self.device) % R
-            self.residual_key[b][:, slots] = keys[:, q:]
-            self.residual_value[b][:, slots] = values[:, q:]
-        self.seq_lengths[b] = L
+        if D != self.head_dim:
+            raise ValueError(f"keys/values must have head_dim {self.head_dim}, got {D}")
+        if L == 0:
+            self.seq_lengths[b] = 0
+        else:
+            self._store(range(self.batch)[b], keys.expand(self.kv_heads, L, D), values.expand(self.kv_heads, L, D))
         self.lengths[b] = L
+
+    def _store(self, b: int, keys: torch.Tensor, values: torch.Tensor) -> None:
+        """Row b becomes keys/values [Hkv, L, D], codes, window and length, in one launch."""
+        _lib.require_device(keys, values, self.residual_key)
+        keys, values = fused_ops.tq_store_rows(keys.unsqueeze(0)), fused_ops.tq_store_rows(values.unsqueeze(0))
+        _, H, L, D = keys.shape
+        R = self.residual_capacity
+        a = _lib.TQStoreArgs()
+        a.dtype, a.key_format = _lib.dtype_code(torch.bfloat16), 0
+        a.batch, a.row0, a.rows = self.batch, b, 1
+        a.kv_heads, a.head_dim, a.tokens, a.capacity, a.residual_capacity = H, D, L, self.capacity, R
+        a.key_bits = a.value_bits = self.bits
+        a.value_group_size = self.value_group_size
+        a.new_key, a.new_value = keys.data_ptr(), values.data_ptr()
+        a.key_stride_row, a.key_stride_head, a.key_stride_token, _ = keys.stride()
+        a.value_stride_row, a.value_stride_head, a.value_stride_token, _ = values.stride()
+        a.key_codes, a.key_norms = self.key_codes.data_ptr(), self.key_norms.data_ptr()
+        a.value_data, a.value_scales, a.value_zeros = (self.value_data.data_ptr(), self.value_scales.data_ptr(),
+                                                       self.value_zeros.data_ptr())
+        a.residual_key, a.residual_value = self.residual_key.data_ptr(), self.residual_value.data_ptr()
+        a.seq_out = self.seq_lengths.data_ptr()
+        a.max_leaving, a.max_fill = max(0, L - R), min(R, L)
+        a.signs, a.thresholds = self.qn.signs.data_ptr(), self.qn.thresholds.data_ptr()
+        _lib.call("anna_mi_tq_store", ctypes.byref(a), _lib.stream_of(keys))
 
     def append(self, keys: torch.Tensor, values: torch.Tensor) -> None:
         """One token per sequence: keys/values bf16 [B, Hkv, D]."""

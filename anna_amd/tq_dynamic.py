@@ -26,6 +26,8 @@ depend on token order, and while a sequence is shorter than the window its token
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib
@@ -36,10 +38,9 @@ from .turboquant import (
     TurboQuantKeyState,
     TurboQuantKVRow,
     _next_capacity,
-    _quantize_turboquant_keys,
     _require_rocm,
     _resolve_value_group_size,
-    dequantize_turboquant_keys,
+    get_turboquant_ip_quantizer,
     get_turboquant_quantizer,
     quantize_turboquant_values,
 )
@@ -58,7 +59,15 @@ class _LayerSlab:
         self.value_group_size = value_group_size or _resolve_value_group_size(head_dim)
         self.capacity = 0
         self.lengths = [0] * batch
+        # device lengths: an append reads one array and writes the other, which becomes seq_lengths
         self.seq_lengths = torch.zeros((batch,), dtype=torch.int32, device=device)
+        self._next_lengths = torch.zeros_like(self.seq_lengths)
+        # one launch per append (anna_mi_tq_store) wherever the keys' rotation is the Hadamard one;
+        # other head_dims (TQ-MSE keys, or no token past the window) go quantizer by quantizer
+        self._qn = None
+        if head_dim in (64, 128, 256, 512, 1024) and dtype in (torch.bfloat16, torch.float16, torch.float32):
+            get = get_turboquant_ip_quantizer if key_quantizer == "ip" else get_turboquant_quantizer
+            self._qn = get(head_dim=head_dim, bits=bits, device=device)
         B, H, R, D = batch, heads, residual_len, head_dim
         self.rk = torch.zeros((B, H, R, D), dtype=dtype, device=device)
         self.rv = torch.zeros((B, H, R, D), dtype=dtype, device=device)
@@ -98,20 +107,14 @@ class _LayerSlab:
         self.capacity = cap
 
     def _quantize(self, keys: torch.Tensor, values: torch.Tensor) -> dict[str, torch.Tensor]:
-        """keys/values [n, D] -> the per-token fields, each [n, ...]."""
+        """keys/values [n, D] -> the per-token fields, each [n, ...] (TQ-MSE keys of a dense rotation)."""
         n, D = keys.shape
+        if self.key_quantizer == "ip":  # raises: the quantizer takes the head_dims of the one-launch append
+            get_turboquant_ip_quantizer(head_dim=D, bits=self.bits, device=self.device)
         v = quantize_turboquant_values(values.reshape(n, 1, D), bits=self.bits, group_size=self.value_group_size)
-        out = {"vdata": v.data.reshape(n, -1), "vscales": v.scales.reshape(n, -1), "vzeros": v.zeros.reshape(n, -1)}
-        if self.key_quantizer == "ip":
-            st = _quantize_turboquant_keys(keys.reshape(n, 1, D), bits=self.bits, device=self.device)
-            out.update(kidx=st.mse_indices.reshape(n, D), knorms=st.norms.reshape(n), kqjl=st.qjl_signs.reshape(n, D),
-                       krn=st.residual_norms.reshape(n),
-                       kdense=dequantize_turboquant_keys(st, bits=self.bits, device=self.device,
-                                                         dtype=self.dtype).reshape(n, D))
-        else:
-            codes, norms = get_turboquant_quantizer(head_dim=D, bits=self.bits, device=self.device).quantize(keys)
-            out.update(kcodes=codes, knorms=norms)
-        return out
+        codes, norms = get_turboquant_quantizer(head_dim=D, bits=self.bits, device=self.device).quantize(keys)
+        return {"vdata": v.data.reshape(n, -1), "vscales": v.scales.reshape(n, -1), "vzeros": v.zeros.reshape(n, -1),
+                "kcodes": codes, "knorms": norms}
 
     def store_range(self, b: int, start: int, keys: torch.Tensor, values: torch.Tensor) -> None:
         """Quantize keys/values [H, t, D] of sequence b into its slots start..start+t-1."""
@@ -140,25 +143,81 @@ class _LayerSlab:
         return self.rk[b][:, slots], self.rv[b][:, slots]
 
     # ---- appends
-    def append(self, keys: torch.Tensor, values: torch.Tensor) -> None:
+    def append(self, keys: torch.Tensor, values: torch.Tensor) -> torch.Tensor:
         """keys/values [B, H, T, D]: T new tokens for every sequence (reference row append,
-        turboquant.py:1027-1140, for all rows)."""
-        B, H, T, D = keys.shape
-        if T == 1 and all(n >= self.R for n in self.lengths):
-            # decode step: each sequence's oldest window token (slot L % R) is quantized into
-            # slot L - R and the new token takes its place in the ring
-            self._grow(max(self.lengths) - self.R + 1)
-            rows = torch.arange(B, device=self.device)
-            lens = self.seq_lengths.long()
-            ring = lens % self.R
-            self.store_scatter(rows, lens - self.R, self.rk[rows, :, ring], self.rv[rows, :, ring])
-            self.rk[rows, :, ring] = keys[:, :, 0]
-            self.rv[rows, :, ring] = values[:, :, 0]
+        turboquant.py:1027-1140, for all rows).  Returns the lengths before (device int64 [B])."""
+        return self._append(0, keys, values)
+
+    def append_row(self, b: int, keys: torch.Tensor, values: torch.Tensor) -> None:
+        """keys/values [H, T, D]: T new tokens for sequence b."""
+        self._append(range(self.batch)[b], keys.unsqueeze(0), values.unsqueeze(0))
+
+    def _append(self, row0: int, keys: torch.Tensor, values: torch.Tensor) -> torch.Tensor:
+        rows, _, T, _ = keys.shape
+        if self._qn is None:
+            past = self.seq_lengths.long()
+            if rows == self.batch and T == 1 and all(n >= self.R for n in self.lengths):
+                self._append_step(keys, values)
+            else:
+                for i in range(rows):
+                    self._append_row(row0 + i, keys[i], values[i])
+            self.seq_lengths[row0:row0 + rows] += T
         else:
-            for b in range(B):
-                self._append_row(b, keys[b], values[b])
-        self.lengths = [n + T for n in self.lengths]
-        self.seq_lengths += T
+            past = self._store(row0, keys, values)
+        for b in range(row0, row0 + rows):
+            self.lengths[b] += T
+        return past
+
+    def _store(self, row0: int, keys: torch.Tensor, values: torch.Tensor) -> torch.Tensor:
+        """The append in one launch (anna_mi_tq_store)."""
+        rows, H, T, D = keys.shape
+        R = self.R
+        lens = self.lengths[row0:row0 + rows]
+        self._grow(max(n + T - R for n in lens))
+        _lib.require_device(keys, values, self.rk)
+        keys, values = fused_ops.tq_store_rows(keys), fused_ops.tq_store_rows(values)
+        qn, ip, C = self._qn, self.key_quantizer == "ip", self.capacity
+        past = torch.empty((self.batch,), dtype=torch.int64, device=self.device)
+        a = _lib.TQStoreArgs()
+        a.dtype, a.key_format = _lib.dtype_code(self.dtype), int(ip)
+        a.batch, a.row0, a.rows = self.batch, row0, rows
+        a.kv_heads, a.head_dim, a.tokens, a.capacity, a.residual_capacity = H, D, T, C, R
+        a.key_bits = a.value_bits = self.bits
+        a.value_group_size = self.value_group_size
+        a.new_key, a.new_value = keys.data_ptr(), values.data_ptr()
+        a.key_stride_row, a.key_stride_head, a.key_stride_token, _ = keys.stride()
+        a.value_stride_row, a.value_stride_head, a.value_stride_token, _ = values.stride()
+        if C > 0:
+            a.key_norms = self.knorms.data_ptr()
+            a.value_data, a.value_scales, a.value_zeros = (self.vdata.data_ptr(), self.vscales.data_ptr(),
+                                                           self.vzeros.data_ptr())
+            if ip:
+                a.key_codes, a.key_signs = self.kidx.data_ptr(), self.kqjl.data_ptr()
+                a.key_residual_norms, a.key_dense = self.krn.data_ptr(), self.kdense.data_ptr()
+            else:
+                a.key_codes = self.kcodes.data_ptr()
+        a.residual_key, a.residual_value = self.rk.data_ptr(), self.rv.data_ptr()
+        a.seq_in, a.seq_out, a.past_out = self.seq_lengths.data_ptr(), self._next_lengths.data_ptr(), past.data_ptr()
+        a.max_leaving = max(max(0, n + T - R) - max(0, n - R) for n in lens)
+        a.max_fill = max(max(0, min(R, n + T) - n) for n in lens)
+        a.signs, a.thresholds = qn.signs.data_ptr(), qn.thresholds.data_ptr()
+        if ip:
+            a.centroids, a.gaussian, a.gaussian_t = (qn.centroids.data_ptr(), qn.gaussian.data_ptr(),
+                                                     qn.gaussian_t.data_ptr())
+        _lib.call("anna_mi_tq_store", ctypes.byref(a), _lib.stream_of(keys))
+        self.seq_lengths, self._next_lengths = self._next_lengths, self.seq_lengths
+        return past
+
+    def _append_step(self, keys: torch.Tensor, values: torch.Tensor) -> None:
+        """A decode step of full windows: each sequence's oldest window token (slot L % R) is
+        quantized into slot L - R and the new token takes its place in the ring."""
+        self._grow(max(self.lengths) - self.R + 1)
+        rows = torch.arange(self.batch, device=self.device)
+        lens = self.seq_lengths.long()
+        ring = lens % self.R
+        self.store_scatter(rows, lens - self.R, self.rk[rows, :, ring], self.rv[rows, :, ring])
+        self.rk[rows, :, ring] = keys[:, :, 0]
+        self.rv[rows, :, ring] = values[:, :, 0]
 
     def _append_row(self, b: int, keys: torch.Tensor, values: torch.Tensor) -> None:
         H, T, D = keys.shape
@@ -374,11 +433,12 @@ class TurboQuantDynamicCache:
         return len(self.layer_lengths[0]) if self.layer_lengths else 0
 
     def get_seq_lengths(self, *, device=None) -> torch.Tensor:
-        lengths = []
-        for b in range(self.get_batch_size()):
-            lengths.append(next((self.layer_lengths[i][b] for i in range(self.num_layers)
-                                 if self.layer_lengths[i][b] > 0), 0))
-        return torch.tensor(lengths, dtype=torch.long, device=device)
+        return torch.tensor(self._row_lengths(), dtype=torch.long, device=device)
+
+    def _row_lengths(self) -> list[int]:
+        """Length of each sequence: that of the first layer that holds any of it."""
+        return [next((lens[b] for lens in self.layer_lengths if lens[b] > 0), 0)
+                for b in range(self.get_batch_size())]
 
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int, *,
                require_dense_cache: bool = True):
@@ -391,7 +451,6 @@ class TurboQuantDynamicCache:
         B, H, T, D = key_states.shape
         self._ensure_batch_size(B)
         _require_rocm(key_states, "TurboQuantDynamicCache")
-        past_lengths = torch.tensor(self.layer_lengths[layer_idx], device=key_states.device, dtype=torch.long)
         slab = self._slabs[layer_idx]
         if slab is None:
             slab = _LayerSlab(batch=B, heads=H, head_dim=D, dtype=key_states.dtype, device=key_states.device,
@@ -403,9 +462,11 @@ class TurboQuantDynamicCache:
             raise ValueError(f"TurboQuantKVRow shape mismatch: expected heads={slab.heads} head_dim={slab.head_dim}, "
                              f"got {tuple(key_states.shape[1:])}")
         if T > 0:
-            slab.append(key_states.to(dtype=slab.dtype).detach(), value_states.to(dtype=slab.dtype).detach())
+            past_lengths = slab.append(key_states.to(dtype=slab.dtype).detach(), value_states.to(dtype=slab.dtype).detach())
+        else:
+            past_lengths = slab.seq_lengths.long()
         self.layer_lengths[layer_idx] = list(slab.lengths)
-        self.seen_tokens = max(self.get_seq_lengths().tolist(), default=0)
+        self.seen_tokens = max(self._row_lengths(), default=0)
         if not require_dense_cache:
             return None, None, past_lengths
         rows = [r.materialize(device=key_states.device, dtype=key_states.dtype)
@@ -426,9 +487,7 @@ class TurboQuantDynamicCache:
         T = int(key_states.shape[1])
         if T == 0:
             return
-        slab._append_row(batch_idx, key_states.to(dtype=slab.dtype).detach(), value_states.to(dtype=slab.dtype).detach())
-        slab.lengths[batch_idx] += T
-        slab.seq_lengths[batch_idx] += T
+        slab.append_row(batch_idx, key_states.to(dtype=slab.dtype).detach(), value_states.to(dtype=slab.dtype).detach())
         self.layer_lengths[layer_idx] = list(slab.lengths)
 
     def turboquant_single_token_decode_attention(self, layer_idx: int, query_states: torch.Tensor, *,

@@ -398,6 +398,52 @@ typedef struct {
 int64_t anna_mi_sizeof_tq_rows_append_args(void);
 int anna_mi_tq_rows_append(const anna_mi_tq_rows_append_args* args, void* stream);
 
+/* `tokens` tokens of each of the rows row0 .. row0 + rows - 1 of a layer join its slab, in one
+ * launch: Qwen3DynamicCache._update_turboquant_layer looping TurboQuantKVRow.append (ops.py:618-661,
+ * turboquant.py:1027-1140), for prompts and decode steps alike.  A row of length L keeps its newest
+ * R tokens in the ring (token j at slot j % R); the tokens that leave it are quantized into slot j.
+ * Keys: TQ-MSE codes + fp16 norms (key_format 0, as anna_mi_tq_hadamard_quantize) or the
+ * inner-product state and its reconstruction in the cache dtype (key_format 1, bit for bit as
+ * anna_mi_tq_ip_quantize and anna_mi_tq_ip_dequant).  Values: min/max groups (as
+ * anna_mi_tq_values_quantize).  Slots past `capacity` are not written. */
+typedef struct {
+  int dtype; /* new tokens, ring, value scales/zeros, key reconstruction */
+  int key_format;
+  int64_t batch, row0, rows; /* rows of the slab; the ones that grow */
+  int64_t kv_heads, head_dim, tokens, capacity, residual_capacity;
+  int key_bits, value_bits;
+  int64_t value_group_size;
+  const void* new_key;   /* (row, head, token, d) at the strides below (elements), d contiguous */
+  const void* new_value;
+  int64_t key_stride_row, key_stride_head, key_stride_token;
+  int64_t value_stride_row, value_stride_head, value_stride_token;
+  uint8_t* key_codes;          /* [B, H, capacity, D * sbits / 8], or byte indices [B, H, capacity, D] */
+  void* key_norms;             /* [B, H, capacity]: fp16, or fp32 for key_format 1 */
+  uint8_t* key_signs;          /* key_format 1: [B, H, capacity, D] 0 / 1 */
+  float* key_residual_norms;   /* key_format 1: [B, H, capacity] */
+  void* key_dense;             /* key_format 1: [B, H, capacity, D] */
+  uint8_t* value_data;         /* [B, H, capacity, D * sbits / 8] */
+  void* value_scales;          /* [B, H, capacity, D / group] */
+  void* value_zeros;
+  void* residual_key;          /* [B, H, R, D] */
+  void* residual_value;
+  const int32_t* seq_in;       /* device [B] lengths before, or NULL: the rows start empty */
+  int32_t* seq_out;            /* device [B] lengths after (another array; with seq_in NULL only the rows' own) */
+  int64_t* past_out;           /* device [B] lengths before as int64, or NULL */
+  int64_t max_leaving;         /* at least the tokens that leave any one row's window */
+  int64_t max_fill;            /* at least the ring slots any one row fills for the first time */
+  const float* signs;          /* Hadamard signs [D] */
+  const float* thresholds;
+  const float* centroids;      /* key_format 1 */
+  const float* gaussian;       /* key_format 1: G [D, D] and its transpose */
+  const float* gaussian_t;
+  int value_lane_groups;       /* set by the library */
+  float k0;                    /* set by the library */
+} anna_mi_tq_store_args;
+
+int64_t anna_mi_sizeof_tq_store_args(void);
+int anna_mi_tq_store(const anna_mi_tq_store_args* args, void* stream);
+
 typedef struct {
   int64_t kv_heads, head_dim, tokens;
   const uint16_t* keys;             /* bf16, element (h, t, d) at h * stride_head + t * stride_token + d */

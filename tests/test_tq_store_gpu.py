@@ -1,0 +1,132 @@
+"""The one-launch append of the dynamic cache (anna_mi_tq_store) against rows that quantize token by
+token: codes, norms, signs, reconstruction, values, window and lengths, bit for bit.
+
+The rows (TurboQuantKVRow) run the separate quantizers, which their own tests hold to the oracle.
+"""
+
+import pytest
+import torch
+
+from anna_amd.tq_cache import TurboQuantBatchCache
+from anna_amd.tq_dynamic import TurboQuantDynamicCache
+from anna_amd.turboquant import TurboQuantKVRow
+
+pytestmark = pytest.mark.gpu
+
+
+def same(a, b):
+    a, b = a.contiguous(), b.contiguous()
+    assert a.shape == b.shape and a.dtype == b.dtype
+    assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def check_row(cache, b, row):
+    slab, n = cache._slabs[0], row.quantized_length
+    got = cache.turboquant_rows[0][b]
+    assert (got.length, got.quantized_length) == (row.length, n)
+    pairs = [("vdata", "_vdata"), ("vscales", "_vscales"), ("vzeros", "_vzeros"), ("knorms", "_knorms")]
+    if slab.key_quantizer == "ip":
+        pairs += [("kidx", "_kcodes"), ("kqjl", "_kqjl"), ("krn", "_krn"), ("kdense", "_kdense")]
+    else:
+        pairs += [("kcodes", "_kcodes")]
+    if n:
+        for mine, theirs in pairs:
+            same(getattr(slab, mine)[b, :, :n], getattr(row, theirs)[:, :n])
+    wk, wv = slab.window(b)
+    same(wk, row._residual_keys)
+    same(wv, row._residual_values)
+
+
+# chunks that stay inside the window, fill it exactly, cross it from part full, wrap it more than
+# once, and single tokens; 17 x 2 heads vectors end inside a tile of 16
+PLANS = [(5, 27, 1, 1), (40, 1, 1), (3, 30, 200, 1, 77), (32, 1, 33, 64)]
+
+
+@pytest.mark.parametrize("head_dim,bits,key_quantizer,dtype,group", [
+    (64, 4, "ip", torch.bfloat16, None), (128, 3, "ip", torch.float16, 16), (256, 2, "ip", torch.bfloat16, None),
+    (512, 4, "ip", torch.float32, 64), (1024, 4, "ip", torch.bfloat16, 512), (128, 4, "mse", torch.bfloat16, None),
+    (256, 2, "mse", torch.float32, 4), (64, 3, "mse", torch.float16, 1), (192, 4, "mse", torch.bfloat16, None),
+    (1024, 2, "mse", torch.bfloat16, 1024),
+])
+@pytest.mark.parametrize("plan", PLANS)
+def test_store_matches_rows(gpu, head_dim, bits, key_quantizer, dtype, group, plan):
+    torch.manual_seed(head_dim + bits)
+    batch, heads, window = 3, 2, 32
+    cache = TurboQuantDynamicCache(1, kv_cache_quant_bits=bits, kv_cache_residual_len=window,
+                                   key_quantizer=key_quantizer, value_group_size=group)
+    rows = [TurboQuantKVRow(bits=bits, residual_len=window, value_group_size=group, key_quantizer=key_quantizer)
+            for _ in range(batch)]
+    total = 0
+    for i, t in enumerate(plan):
+        # [B, T, H, D] transposed: strides of the attention's own layout
+        k = torch.randn(batch, t, heads, head_dim, device=gpu).to(dtype).transpose(1, 2)
+        v = torch.randn(batch, t, heads, head_dim, device=gpu).to(dtype).transpose(1, 2)
+        _, _, past = cache.update(k, v, 0, require_dense_cache=False)
+        assert past.dtype == torch.int64 and past.tolist() == [r.length for r in rows]
+        for b in range(batch):
+            rows[b].append(k[b], v[b])
+        if i == 1:  # one sequence moves ahead of the others
+            ek, ev = (torch.randn(heads, 7, head_dim, device=gpu).to(dtype) for _ in range(2))
+            cache.append_row(0, 1, ek, ev)
+            rows[1].append(ek, ev)
+        total += t
+        for b in range(batch):
+            check_row(cache, b, rows[b])
+        assert cache._slabs[0].seq_lengths.tolist() == [r.length for r in rows]
+
+
+def test_large_tiles_match_small_ones(gpu):
+    """A prompt long enough for the tiles of 64 vectors equals the same tokens in two chunks of the
+    tiles of 16 (both end inside a tile)."""
+    torch.manual_seed(3)
+    for head_dim in (64, 128, 256, 512):
+        k, v = (torch.randn(1, 2, 4321, head_dim, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        caches = [TurboQuantDynamicCache(1, kv_cache_quant_bits=4) for _ in range(2)]
+        caches[0].update(k, v, 0, require_dense_cache=False)
+        for a, z in ((0, 3000), (3000, 4321)):
+            caches[1].update(k[:, :, a:z], v[:, :, a:z], 0, require_dense_cache=False)
+        one, two = (c._slabs[0] for c in caches)
+        n = 4321 - 128
+        for name in ("kidx", "knorms", "kqjl", "krn", "kdense", "vdata", "vscales", "vzeros"):
+            same(getattr(one, name)[:, :, :n], getattr(two, name)[:, :, :n])
+        same(one.rk, two.rk)
+        same(one.rv, two.rv)
+
+
+@pytest.mark.parametrize("head_dim,bits", [(128, 4), (64, 2), (512, 3)])
+@pytest.mark.parametrize("length", [1, 128, 129, 700])
+def test_rows_cache_load_equals_appends(gpu, head_dim, bits, length):
+    """load_sequence over a row that held other tokens leaves what as many appends leave."""
+    torch.manual_seed(length)
+    batch, heads = 2, 2
+    caches = [TurboQuantBatchCache(batch=batch, kv_heads=heads, q_heads=2 * heads, capacities=[640, 700],
+                                   head_dim=head_dim, bits=bits) for _ in range(2)]
+    k, v = (torch.randn(length, batch, heads, head_dim, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+    for t in range(length):
+        caches[0].append(k[t], v[t])
+    caches[1].load_sequence(1, *(torch.randn(heads, 300, head_dim, device=gpu, dtype=torch.bfloat16) for _ in range(2)))
+    for b in range(batch):
+        caches[1].load_sequence(b, k[:, b].transpose(0, 1), v[:, b].transpose(0, 1))
+    one, two = caches
+    assert one.lengths == two.lengths == one.seq_lengths.tolist() == two.seq_lengths.tolist()
+    n, r = max(0, length - 128), min(length, 128)
+    for name in ("key_codes", "key_norms", "value_data", "value_scales", "value_zeros"):
+        same(getattr(one, name)[:, :, :n], getattr(two, name)[:, :, :n])
+    for name in ("residual_key", "residual_value"):
+        same(getattr(one, name)[:, :, :r], getattr(two, name)[:, :, :r])
+
+
+def test_store_refusals(gpu):
+    cache = TurboQuantDynamicCache(1, kv_cache_residual_len=16)
+    good = torch.randn(2, 2, 20, 128, device=gpu, dtype=torch.bfloat16)
+    cache.update(good, good, 0)
+    with pytest.raises(RuntimeError):
+        cache.update(good.cpu(), good.cpu(), 0)
+    with pytest.raises(IndexError):
+        cache.append_row(0, 2, good[0], good[0])
+    # a head_dim the inner-product quantizer does not take is refused once tokens leave the window
+    other = TurboQuantDynamicCache(1, kv_cache_residual_len=16)
+    odd = torch.randn(1, 2, 12, 96, device=gpu, dtype=torch.bfloat16)
+    other.update(odd, odd, 0, require_dense_cache=False)
+    with pytest.raises(ValueError):
+        other.update(odd, odd, 0, require_dense_cache=False)
