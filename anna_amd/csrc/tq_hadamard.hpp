@@ -146,6 +146,30 @@ __device__ __forceinline__ void sumsq_wave_n(const float (&x)[NV][E], float (&ou
   for (int n = 0; n < NV; ++n) out[n] = out[n] + xor_lane<32>(out[n]);
 }
 
+// code = number of thresholds t_j (nthr <= 64 of them) with y >= fl(t_j * norm).  The thresholds come
+// from a register of the wave, one per lane, and the loop over them is the outer one: read from memory
+// inside the loop over elements, every comparison waited for a scalar load (8,192 vectors of 128 at
+// 4 bits, keys and values: 16.4 -> 9.9 us).
+template <int NV, int E>
+__device__ __forceinline__ void count_thresholds_n(const float (&y)[NV][E], const float* __restrict__ thr, int nthr,
+                                                   const float (&nrm)[NV], uint32_t (&code)[NV][E]) {
+  const int lane = threadIdx.x & 63;
+  const float mine = thr[lane < nthr ? lane : nthr - 1];
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int e = 0; e < E; ++e) code[n][e] = 0;
+  for (int j = 0; j < nthr; ++j) {
+    const float t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), j));
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const float tn = __fmul_rn(t, nrm[n]);
+#pragma unroll
+      for (int e = 0; e < E; ++e) code[n][e] += y[n][e] >= tn ? 1u : 0u;
+    }
+  }
+}
+
 // Quantize NV vectors of the wave (lane's E elements each, fp32 values of the input): the lane's
 // E codes per vector (1 byte each) and the norms (all lanes).
 template <int NV, int E>
@@ -169,12 +193,8 @@ __device__ __forceinline__ void hadamard_codes_wave_n(const float (&x)[NV][E], c
 #pragma unroll
   for (int n = 0; n < NV; ++n)
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const float y = v[n][e] * inv;
-      uint32_t c = 0;
-      for (int j = 0; j < nthr; ++j) c += y >= __fmul_rn(thr[j], nrm[n]) ? 1u : 0u;
-      code[n][e] = c;
-    }
+    for (int e = 0; e < E; ++e) v[n][e] = v[n][e] * inv;
+  count_thresholds_n<NV, E>(v, thr, nthr, nrm, code);
 }
 
 template <int E>

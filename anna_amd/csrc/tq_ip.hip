@@ -72,13 +72,19 @@ __device__ __forceinline__ void matvec_wave_n(const float* __restrict__ M, const
 template <int XDT, int E, int TV>
 __global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_quantize_kernel(
     const typename Elem<XDT>::T* __restrict__ x, int64_t nvec, int64_t xs, const float* __restrict__ signs,
-    const float* __restrict__ thr, const float* __restrict__ cent, int nthr, const float* __restrict__ gt,
+    const float* __restrict__ thr, const float* __restrict__ cent, int bits, const float* __restrict__ gt,
     uint8_t* __restrict__ idx_out, uint8_t* __restrict__ qjl_out, float* __restrict__ norm_out,
     float* __restrict__ rn_out) {
   extern __shared__ __attribute__((aligned(16))) float ip_lds[];
   constexpr int D = 64 * E, VW = TV / IP_WAVES, NB = VW < 4 ? VW : 4;
   const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t v0 = (int64_t)blockIdx.x * TV + wave * VW;
+  IpMatrix<E> m;
+  if constexpr (ip_whole<E, TV>()) {
+    m.load(gt, wave);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const float ctab = ip_centroid_table(cent, bits);
 #pragma unroll
   for (int n0 = 0; n0 < VW; n0 += NB) {
     float xv[NB][E], rho[NB][E], nrm[NB], rn[NB];
@@ -89,7 +95,7 @@ __global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_quantize_kernel(
 #pragma unroll
       for (int e = 0; e < E; ++e) xv[n][e] = Elem<XDT>::load(x, v * xs + lane * E + e);
     }
-    ip_mse_stage<NB, E>(xv, signs, thr, cent, nthr, code, nrm, rho, rn);
+    ip_mse_stage<NB, E>(xv, signs, thr, ctab, (1 << (bits - 1)) - 1, code, nrm, rho, rn);
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
       const int64_t v = v0 + n0 + n;
@@ -105,7 +111,7 @@ __global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_quantize_kernel(
       }
     }
   }
-  ip_signs<E, TV>(gt, ip_lds, wave);
+  ip_signs<E, TV>(gt, m, nullptr, ip_lds, wave);
 #pragma unroll
   for (int n = 0; n < VW; ++n) {
     const int64_t v = v0 + n;
@@ -120,11 +126,17 @@ template <int ODT, int E, int TV>
 __global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_dequant_kernel(
     const uint8_t* __restrict__ idx, const uint8_t* __restrict__ qjl, const float* __restrict__ norms,
     const float* __restrict__ rn, int64_t nvec, const float* __restrict__ signs, const float* __restrict__ cent,
-    const float* __restrict__ g, float k0, typename Elem<ODT>::T* __restrict__ out, int64_t os) {
+    const float* __restrict__ g, int bits, float k0, typename Elem<ODT>::T* __restrict__ out, int64_t os) {
   extern __shared__ __attribute__((aligned(16))) float ip_lds[];
   constexpr int D = 64 * E, VW = TV / IP_WAVES;
   const int wave = (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t v0 = (int64_t)blockIdx.x * TV + wave * VW;
+  IpMatrix<E> m;
+  if constexpr (ip_whole<E, TV>()) {
+    m.load(g, wave);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const float ctab = ip_centroid_table(cent, bits);
 #pragma unroll
   for (int n = 0; n < VW; ++n) {
     const int64_t v = v0 + n < nvec ? v0 + n : nvec - 1;
@@ -133,7 +145,7 @@ __global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_dequant_kernel(
     for (int e = 0; e < E; ++e) my[ip_pos(lane * E + e)] = qjl[v * D + lane * E + e] ? 1.f : -1.f;
   }
   __syncthreads();
-  ip_project<E, TV>(g, ip_lds, wave);
+  ip_project<E, TV>(g, m, ip_lds, wave);
   float sg[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) sg[e] = signs[lane * E + e];
@@ -143,7 +155,7 @@ __global__ __launch_bounds__(64 * IP_WAVES) void tq_ip_dequant_kernel(
     if (v >= nvec) break;
     float c[E], o[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) c[e] = cent[idx[v * D + lane * E + e]];
+    for (int e = 0; e < E; ++e) c[e] = ip_centroid(ctab, idx[v * D + lane * E + e]);
     ip_reconstruct<E>(ip_lds + (wave * VW + n) * IP_ROW<E>, c, k0 * rn[v], norms[v], sg, lane, o);
 #pragma unroll
     for (int e = 0; e < E; ++e) out[v * os + lane * E + e] = Elem<ODT>::cvt(o[e]);
@@ -257,9 +269,6 @@ void dispatch_e(int64_t D, F&& go) {
 
 bool ip_dim_ok(int64_t D) { return D == 64 || D == 128 || D == 256 || D == 512 || D == 1024; }
 
-// Tiles of 16 while that leaves at most 32 vectors per compute unit, else the large tile.
-bool ip_small(int64_t nvec) { return nvec < 256 * 32; }
-
 template <class K>
 int ip_raise_lds(K kern, size_t lds, const char* what) {
   ANNA_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess,
@@ -292,7 +301,6 @@ extern "C" int anna_mi_tq_ip_quantize(const void* x, int x_dtype, int64_t nvec, 
   ANNA_CHECK(ip_dim_ok(D), "anna_mi_tq_ip_quantize: head_dim must be a power of two in [64, 1024]");
   ANNA_CHECK(x_row_stride >= D, "anna_mi_tq_ip_quantize: row stride smaller than head_dim");
   ANNA_CHECK(nvec > 0, "anna_mi_tq_ip_quantize: negative vector count");
-  const int nthr = (1 << (bits - 1)) - 1;
   int rc = ANNA_MI_OK;
   ANNA_DISPATCH_DTYPE(x_dtype, XDT, {
     dispatch_e(D, [&](auto e_tag) {
@@ -304,10 +312,10 @@ extern "C" int anna_mi_tq_ip_quantize(const void* x, int x_dtype, int64_t nvec, 
         rc = ip_raise_lds(kern, lds, "anna_mi_tq_ip_quantize");
         if (rc != ANNA_MI_OK) return;
         hipLaunchKernelGGL(kern, dim3((unsigned)((nvec + TV - 1) / TV)), dim3(64 * IP_WAVES), lds, as_stream(stream),
-                           (const typename Elem<XDT>::T*)x, nvec, x_row_stride, signs, thresholds, centroids, nthr,
+                           (const typename Elem<XDT>::T*)x, nvec, x_row_stride, signs, thresholds, centroids, bits,
                            gaussian_t, mse_indices, qjl_signs, norms, residual_norms);
       };
-      if (ip_small(nvec)) go(std::integral_constant<int, ip_tile(E, true)>{});
+      if (ip_small_tiles(nvec)) go(std::integral_constant<int, ip_tile(E, true)>{});
       else go(std::integral_constant<int, ip_tile(E, false)>{});
     });
   });
@@ -339,10 +347,10 @@ extern "C" int anna_mi_tq_ip_dequant(const uint8_t* mse_indices, const uint8_t* 
         rc = ip_raise_lds(kern, lds, "anna_mi_tq_ip_dequant");
         if (rc != ANNA_MI_OK) return;
         hipLaunchKernelGGL(kern, dim3((unsigned)((nvec + TV - 1) / TV)), dim3(64 * IP_WAVES), lds, as_stream(stream),
-                           mse_indices, qjl_signs, norms, residual_norms, nvec, signs, centroids, gaussian, ip_k0(D),
+                           mse_indices, qjl_signs, norms, residual_norms, nvec, signs, centroids, gaussian, bits, ip_k0(D),
                            (typename Elem<ODT>::T*)out, out_row_stride);
       };
-      if (ip_small(nvec)) go(std::integral_constant<int, ip_tile(E, true)>{});
+      if (ip_small_tiles(nvec)) go(std::integral_constant<int, ip_tile(E, true)>{});
       else go(std::integral_constant<int, ip_tile(E, false)>{});
     });
   });

@@ -14,11 +14,15 @@
 // another, so no workgroup can see a length another has already raised.
 //
 // What bounds it.  Inner-product keys: the two D x D fp32 products of a vector (4 D^2 flops) on the
-// matrix cores -- 16,128 vectors of D = 256 are 4.2 GFLOP, 27 us at the fp32 matrix rate.  Few
-// vectors (a decode step): one tile of 16, bound by the latency of reading the matrix twice from
-// L2.  TQ-MSE keys and values: bytes.  A step of 8 sequences (D = 128, 2 KV heads, 4 bits) took
-// ~30 launches and 370 us before this kernel; the prompt of 2 x 8192 tokens (D = 256) ran the
-// quantizers at 4 vectors per wave with the matrix re-read from L2 by every wave.
+// matrix cores.  2 x 8064 leaving tokens of 2 KV heads, D = 256: 125 us, of which the products are
+// 55 us at the fp32 matrix rate and 70 us as measured (the call without them: 56 us; keys only: 121
+// us); the transforms before and after run in the same workgroups and overlap with them only across
+// the two workgroups of a compute unit.  Few vectors (a decode step): one tile of 16, bound by one
+// compute unit's fetch of the two matrices and its matrix rate (2 x 2 vectors, D = 256: 27 us with
+// the caches flushed between calls, 45 us before the matrices were loaded whole; 8 x 2 vectors,
+// D = 128: 15 us).  TQ-MSE keys and values: transform and min/max arithmetic (8,192 vectors of 128
+// at 4 bits, keys and values: 9.3 us).  A step of 8 sequences (D = 128, 2 KV heads, 4 bits) was ~30
+// launches and 370 us before this kernel.
 #include <math.h>
 
 #include <type_traits>
@@ -118,6 +122,12 @@ __device__ __forceinline__ void store_ip_keys(const anna_mi_tq_store_args& a, co
   constexpr int CW = E <= 8 ? 1 : 2;  // words of 4-bit codes per vector and lane
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int nthr = (1 << (a.key_bits - 1)) - 1;
+  IpMatrix<E> m;
+  if constexpr (ip_whole<E, TV>()) {
+    m.load(a.gaussian_t, wave);
+    __builtin_amdgcn_sched_barrier(0);  // before anything waits
+  }
+  const float ctab = ip_centroid_table(a.centroids, a.key_bits);
   uint32_t codes[VW][CW];
   float nrm[VW], rnv[VW];
 #pragma unroll
@@ -131,7 +141,7 @@ __device__ __forceinline__ void store_ip_keys(const anna_mi_tq_store_args& a, co
       lv[n] = leaving<T, false>(a, v < g.vectors ? v : g.vectors - 1, v < g.vectors);
       load_elems<XDT, E>(lv[n].src + lane * E, x[n]);
     }
-    ip_mse_stage<NB, E>(x, a.signs, a.thresholds, a.centroids, nthr, cb, nb, rho, rb);
+    ip_mse_stage<NB, E>(x, a.signs, a.thresholds, ctab, nthr, cb, nb, rho, rb);
 #pragma unroll
     for (int n = 0; n < NB; ++n) {
       float* my = lds + (wave * VW + n0 + n) * IP_ROW<E>;
@@ -153,7 +163,7 @@ __device__ __forceinline__ void store_ip_keys(const anna_mi_tq_store_args& a, co
       }
     }
   }
-  ip_signs<E, TV>(a.gaussian_t, lds, wave);
+  ip_signs<E, TV>(a.gaussian_t, m, a.gaussian, lds, wave);
 #pragma unroll
   for (int n = 0; n < VW; ++n) {
     const uint32_t v = blockIdx.x * TV + wave * VW + n;
@@ -165,7 +175,7 @@ __device__ __forceinline__ void store_ip_keys(const anna_mi_tq_store_args& a, co
     for (int e = 0; e < E; ++e) q[e] = lds[(wave * VW + n) * IP_ROW<E> + ip_pos(lane * E + e)] > 0.f ? 1u : 0u;
     store_bytes_wave<E>(q, a.key_signs + lv.slot * D, lane);
   }
-  ip_project<E, TV>(a.gaussian, lds, wave);
+  ip_project<E, TV>(a.gaussian, m, lds, wave);
   float sg[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) sg[e] = a.signs[lane * E + e];
@@ -178,7 +188,7 @@ __device__ __forceinline__ void store_ip_keys(const anna_mi_tq_store_args& a, co
     if (!lv.ok) continue;
     float c[E], out[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) c[e] = a.centroids[(codes[n][e / 8] >> (4 * (e & 7))) & 15u];
+    for (int e = 0; e < E; ++e) c[e] = ip_centroid(ctab, (codes[n][e / 8] >> (4 * (e & 7))) & 15u);
     ip_reconstruct<E>(lds + (wave * VW + n) * IP_ROW<E>, c, k0 * rnv[n], nrm[n], sg, lane, out);
     constexpr int W = E < 8 ? E : 8;
     typedef T TVec __attribute__((ext_vector_type(W)));
@@ -318,7 +328,7 @@ __device__ __forceinline__ void fill_ring(const anna_mi_tq_store_args& a, uint32
 
 // TV: vectors of an inner-product key tile, 0 for TQ-MSE keys
 template <int XDT, int E, int TV>
-__global__ __launch_bounds__(ST_THREADS) void tq_store_kernel(const anna_mi_tq_store_args a, const StoreGrid g) {
+__global__ __launch_bounds__(ST_THREADS, TV > 16 ? 4 : 1) void tq_store_kernel(const anna_mi_tq_store_args a, const StoreGrid g) {
   extern __shared__ __attribute__((aligned(16))) float st_lds[];
   if (blockIdx.x == 0) {
     for (int b = threadIdx.x; b < (int)a.batch; b += ST_THREADS) {
@@ -413,10 +423,7 @@ extern "C" int anna_mi_tq_store(const anna_mi_tq_store_args* ap, void* stream) {
   const int64_t gs = a.value_group_size;
   a.value_lane_groups = gs >= 8 && gs <= ST_VALUE_WAVE_ELEMS && (gs & (gs - 1)) == 0;
   a.k0 = ip_k0(D);
-  // Few vectors: tiles of 16, so that a decode step's work spreads over the chip and a tile's chain
-  // is short; from 64 tiles of 64 per XCD-share on, the large tile reads the matrices a quarter as
-  // often (2 x 8064 tokens of 2 heads, D = 256).
-  const bool small = a.rows * a.kv_heads * a.max_leaving < 256 * 32;
+  const bool small = ip_small_tiles(a.rows * a.kv_heads * a.max_leaving);
   int rc = ANNA_MI_OK;
   ANNA_DISPATCH_DTYPE(a.dtype, XDT, {
     auto go = [&](auto e_tag) {
