@@ -88,6 +88,15 @@ class TQPackArgs(ctypes.Structure):
     ]
 
 
+class TQLoadArgs(ctypes.Structure):
+    """anna_mi_tq_load_args."""
+
+    _fields_ = [
+        ("pack", TQPackArgs), ("length", _I64), ("residual_key", _P), ("residual_value_t", _P),
+        ("residual_capacity", _I64), ("seq_length", _P),
+    ]
+
+
 class TQRowsAppendArgs(ctypes.Structure):
     """anna_mi_tq_rows_append_args."""
 
@@ -121,6 +130,7 @@ PROTOTYPES.update({
     "anna_mi_tq_store": [ctypes.POINTER(TQStoreArgs), _P],
     "anna_mi_tq_rows_append": [ctypes.POINTER(TQRowsAppendArgs), _P],
     "anna_mi_tq_pack_kv": [ctypes.POINTER(TQPackArgs), _P],
+    "anna_mi_tq_load": [ctypes.POINTER(TQLoadArgs), _P],
     "anna_mi_tq_decode": [ctypes.POINTER(TQDecodeArgs), _P],
     "anna_mi_tq_append": [ctypes.POINTER(TQAppendArgs), _P],
     "anna_mi_tq_append_decode": [ctypes.POINTER(TQDecodeArgs), ctypes.POINTER(TQAppendArgs), _P],
@@ -171,6 +181,8 @@ PROTOTYPES.update({
     "anna_mi_int4_gemv_tiled": [_P, _I, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _I, _P, _I64, _I64, _I64, _I64,
                                 _I64, _P, _I, _I64, _P],
     "anna_mi_topk_rows": [_P, _I64, _I64, _I64, _I64, _P, _I, _P, _P],
+    "anna_mi_lm_head_int4_topk_ws": [_P, _I, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _I, _P, _I64, _I64, _I64, _I64,
+                                     _I64, _I64, _P, _P, _P, _P],
     "anna_mi_lm_head_int4_topk": [_P, _I, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _I, _P, _I64, _I64, _I64, _I64,
                                   _I64, _I64, _P, _P, _P, _P],
 })
@@ -183,6 +195,8 @@ RAW_PROTOTYPES: dict[str, tuple] = {
     "anna_mi_sizeof_tq_decode_args": (_I64, []),
     "anna_mi_sizeof_tq_append_args": (_I64, []),
     "anna_mi_sizeof_tq_pack_args": (_I64, []),
+    "anna_mi_sizeof_tq_load_args": (_I64, []),
+    "anna_mi_lm_head_int4_topk_workspace": (_I64, [_I64, _I64]),
     "anna_mi_sizeof_tq_rows_append_args": (_I64, []),
     "anna_mi_sizeof_tq_store_args": (_I64, []),
     "anna_mi_tq_decode_workgroups": (_I64, [_I64, _I64, _P, _I64]),

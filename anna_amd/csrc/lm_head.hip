@@ -711,6 +711,302 @@ __global__ __launch_bounds__(256) void int4_gemv_tiled_lds_kernel(
   }
 }
 
+// ------------------------------------------------------------------ MFMA form (T = 4)
+//
+// A workgroup owns 16 tiles (64 rows of W), its 4 waves a quarter of K each.  A lane's 16-byte load
+// of word w of tile r is word w of the tile's four rows, which are four MFMA operands: lane (r, kq)
+// feeds instruction i with row 4 r + i, so four v_mfma_f32_16x16x32 per 32 k take the 64 rows
+// against up to 16 rows of x at once, and the nibble conversion is paid once for all of them.  (Per
+// row of x the dot2 form above spends six VALU instructions on every 8 weights: 4 rows at
+// V = 151936, K = 2048 took 105 us, this form 42.5; one row 42.7 and 40.0.)  A wave's 16 loads of a
+// pass (512 k) are issued together, after its x, scales and zero points; scale and zero point are
+// applied per 128 k as s (sum x w' - (off + z) sum x) with sum x from an MFMA against ones.
+constexpr int HD_WAVES = 4, HD_ROWS = 64, HD_PASS = 4;  // 128-k blocks per pass of a wave
+
+template <int MP>
+struct HeadLds {
+  u32x4 x[HD_WAVES][16 * HD_PASS * MP];
+  float s[HD_WAVES][HD_PASS * HD_ROWS], z[HD_WAVES][HD_PASS * HD_ROWS];
+  float red[HD_WAVES][MP][HD_ROWS + 1];
+};
+
+// w as exact 16-bit floats of off + q: off = 128 for bf16, 0 for fp16 (1024 + q less 1024: the sums
+// then carry no offset of their own)
+template <int XDT>
+__device__ __forceinline__ u32x4 head_frag(uint32_t w) {
+  u32x4 f = nibbles_to_frag<XDT>(w);
+  if constexpr (XDT == ANNA_MI_F16) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    const f16x2 o = {(_Float16)1024.f, (_Float16)1024.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = __builtin_bit_cast(uint32_t, (f16x2)(__builtin_bit_cast(f16x2, (uint32_t)f[i]) - o));
+  }
+  return f;
+}
+
+// grid (64-row blocks, 16-row blocks of x).  With best_v: also each block's best logit and its index
+// per row of x ([rows][gridDim.x]; ties to the lower index, NaN skipped), for topk_blocks_kernel.
+template <int XDT, int SDT, int MP, bool OUT_F32>
+__global__ __launch_bounds__(64 * HD_WAVES) void int4_head_mfma_kernel(
+    const uint16_t* __restrict__ x, int64_t M_all, int64_t K, int64_t xs, const uint32_t* __restrict__ qw,
+    int64_t tiles, int64_t pc, const typename Elem<SDT>::T* __restrict__ qs, const int8_t* __restrict__ qz,
+    int64_t ss_g, int64_t ss_n, int64_t blocks_per_group, int64_t N, void* __restrict__ y_, int64_t ys,
+    float* __restrict__ best_v, int32_t* __restrict__ best_i) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char head_lds[];
+  HeadLds<MP>& L = *(HeadLds<MP>*)head_lds;
+  constexpr float OFF = XDT == ANNA_MI_BF16 ? 128.0f : 0.0f;
+  constexpr uint32_t ONES = XDT == ANNA_MI_BF16 ? 0x3F803F80u : 0x3C003C00u;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int r = lane & 15, kq = lane >> 4;
+  const int64_t m0 = (int64_t)blockIdx.y * 16;
+  const int M = (int)(M_all - m0 < 16 ? M_all - m0 : 16);
+  x += m0 * xs;
+  const int64_t n0 = (int64_t)blockIdx.x * HD_ROWS;
+  const int64_t tile = (int64_t)blockIdx.x * 16 + r < tiles ? (int64_t)blockIdx.x * 16 + r : tiles - 1;
+  const u32x4* wp = (const u32x4*)qw + tile * pc + kq;
+  const int nblk = (int)(K / 128);
+  const int b_lo = wave * nblk / HD_WAVES, b_hi = (wave + 1) * nblk / HD_WAVES;
+  const int64_t n_mine = n0 + lane < N ? n0 + lane : N - 1;  // lane's row for scales and zero points
+  f32x4 out[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) out[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const u32x4 ones = {ONES, ONES, ONES, ONES};
+  for (int p0 = b_lo; p0 < b_hi; p0 += HD_PASS) {
+    const int nb = b_hi - p0 < HD_PASS ? b_hi - p0 : HD_PASS;
+    // blocks past the wave's share reload its last one with a zero scale
+    float sc[HD_PASS], zp[HD_PASS];
+    typename Elem<SDT>::T sraw[HD_PASS];
+    int8_t zraw[HD_PASS];
+#pragma unroll
+    for (int j = 0; j < HD_PASS; ++j) {
+      const int64_t o = (p0 + (j < nb ? j : nb - 1)) / blocks_per_group * ss_g + n_mine * ss_n;
+      sraw[j] = qs[o];
+      zraw[j] = qz[o];
+    }
+    u32x4 xw[MP];
+    {
+      const int w = lane < 16 * nb ? lane : 16 * nb - 1;
+#pragma unroll
+      for (int m = 0; m < MP; ++m) xw[m] = *(const u32x4*)(x + (m < M ? m : M - 1) * xs + p0 * 128 + w * 8);
+    }
+    u32x4 q[4 * HD_PASS];
+#pragma unroll
+    for (int t = 0; t < 4 * HD_PASS; ++t) {
+      const int j = t / 4 < nb ? t / 4 : nb - 1;
+      q[t] = __builtin_nontemporal_load(wp + (int64_t)(p0 + j) * 16 + (t & 3) * 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < HD_PASS; ++j) {
+      sc[j] = j < nb ? Elem<SDT>::to_f32(sraw[j]) : 0.f;
+      zp[j] = OFF + (float)zraw[j];
+      L.s[wave][j * HD_ROWS + lane] = sc[j];
+      L.z[wave][j * HD_ROWS + lane] = zp[j];
+    }
+#pragma unroll
+    for (int m = 0; m < MP; ++m) L.x[wave][lane * MP + m] = interleave_x(xw[m]);
+    // the staged values are read by this wave only
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int j = 0; j < HD_PASS; ++j) {
+      f32x4 acc[4], sx = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const u32x4 xf = L.x[wave][((4 * j + t) * 4 + kq) * MP + (r & (MP - 1))];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = mfma16<XDT>(head_frag<XDT>(q[4 * j + t][i]), xf, acc[i]);
+        sx = mfma16<XDT>(ones, xf, sx);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x4 sv = *(const f32x4*)&L.s[wave][j * HD_ROWS + (4 * kq + e) * 4];
+        const f32x4 zv = *(const f32x4*)&L.z[wave][j * HD_ROWS + (4 * kq + e) * 4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i][e] = __builtin_fmaf(sv[i], acc[i][e] - zv[i] * sx[e], out[i][e]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the next pass rewrites the staged values
+  }
+  if (r < M && r < MP) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) L.red[wave][r][(4 * kq + e) * 4 + i] = out[i][e];
+  }
+  __syncthreads();
+  const int64_t n = n0 + lane;
+  for (int m = wave; m < M; m += HD_WAVES) {
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < HD_WAVES; ++w) v += L.red[w][m][lane];
+    if (n < N) {
+      if constexpr (OUT_F32) ((float*)y_)[(m0 + m) * ys + n] = v;
+      else ((typename Elem<XDT>::T*)y_)[(m0 + m) * ys + n] = Elem<XDT>::cvt(v);
+    }
+    if (best_v) {
+      const bool use = n < N && v == v;
+      float bv = use ? v : -INFINITY;
+      int32_t bi = use ? (int32_t)n : INT32_MAX;
+      tk_wave_best(bv, bi);
+      if (lane == 0) {
+        best_v[(m0 + m) * gridDim.x + blockIdx.x] = bv;
+        best_i[(m0 + m) * gridDim.x + blockIdx.x] = bi;
+      }
+    }
+  }
+}
+
+// The k best (k <= 32) of a row of logits from its 64-element blocks' bests (C <= 8192 of them): the k
+// best elements lie in the k blocks with the best bests, so one 1024-thread workgroup per row picks
+// those blocks and then the elements among their 64 k.  A pick: the best of each 16-lane row (64 of
+// them), whose k-th best bounds the answer from below; the elements not worse than the bound (a few
+// more than k) go to a list in LDS, and each counts the better ones in it: its rank is its place.
+// The same order as the kernels above, which read every logit back: 4 rows of V = 151936, k = 8:
+// 8.9 + 7.5 us -> 10.4 (rounds of a wave tournament, as there: 16.7); 16 rows, k = 20: 142 -> 14.
+constexpr int TKB_MAX_BLOCKS = 8 * 1024;
+struct TopkLds {
+  float row_v[64], tau_v, top_v[TK_MAX];
+  int32_t row_i[64], tau_i, top_i[TK_MAX], count;
+  float list_v[TKB_MAX_BLOCKS];
+  int32_t list_i[TKB_MAX_BLOCKS];
+};
+
+// The k best of the 1024 threads' NE candidates each (index INT32_MAX: none; indices unique) to
+// L.top, in order; places without a candidate hold -inf, INT32_MAX.
+template <int NE>
+__device__ __forceinline__ void topk_pick(TopkLds& L, const float (&v)[NE], const int32_t (&id)[NE], int k) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float bv = -INFINITY;
+  int32_t bi = INT32_MAX;
+  auto take = [&](float pv, int32_t pi) {
+    if (tk_better(pv, pi, bv, bi)) bv = pv, bi = pi;
+  };
+#pragma unroll
+  for (int j = 0; j < NE; ++j) take(v[j], id[j]);
+  take(__int_as_float(tk_dpp<0xB1>(__float_as_int(bv))), tk_dpp<0xB1>(bi));
+  take(__int_as_float(tk_dpp<0x4E>(__float_as_int(bv))), tk_dpp<0x4E>(bi));
+  take(__int_as_float(tk_dpp<0x141>(__float_as_int(bv))), tk_dpp<0x141>(bi));
+  take(__int_as_float(tk_dpp<0x140>(__float_as_int(bv))), tk_dpp<0x140>(bi));
+  if ((lane & 15) == 0) {
+    L.row_v[wave * 4 + (lane >> 4)] = bv;
+    L.row_i[wave * 4 + (lane >> 4)] = bi;
+  }
+  if (tid < k) L.top_v[tid] = -INFINITY, L.top_i[tid] = INT32_MAX;
+  if (tid == 0) L.count = 0;
+  __syncthreads();
+  if (wave == 0) {
+    const float mv = L.row_v[lane];
+    const int32_t mi = L.row_i[lane];
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+      const float ov = L.row_v[j];
+      const int32_t oi = L.row_i[j];
+      rank += tk_better(ov, oi, mv, mi) || (ov == mv && oi == mi && j < lane);  // (equal only where empty)
+    }
+    if (rank == k - 1) L.tau_v = mv, L.tau_i = mi;
+  }
+  __syncthreads();
+  const float tv = L.tau_v;
+  const int32_t ti = L.tau_i;
+#pragma unroll
+  for (int j = 0; j < NE; ++j) {
+    if (id[j] != INT32_MAX && !tk_better(tv, ti, v[j], id[j])) {
+      const int at = atomicAdd(&L.count, 1);
+      L.list_v[at] = v[j], L.list_i[at] = id[j];
+    }
+  }
+  __syncthreads();
+  const int n = L.count;
+  for (int c = tid; c < n; c += 1024) {
+    const float mv = L.list_v[c];
+    const int32_t mi = L.list_i[c];
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < n; ++j) rank += tk_better(L.list_v[j], L.list_i[j], mv, mi);
+    if (rank < k) L.top_v[rank] = mv, L.top_i[rank] = mi;
+  }
+  __syncthreads();
+}
+
+template <int ODT>
+__global__ __launch_bounds__(1024) void topk_blocks_kernel(const float* __restrict__ logits, int64_t V, int64_t ld,
+                                                           const float* __restrict__ best_v,
+                                                           const int32_t* __restrict__ best_i, int64_t C, int k,
+                                                           typename Elem<ODT>::T* __restrict__ out_v,
+                                                           int64_t* __restrict__ out_i) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char tkb_lds[];
+  TopkLds& L = *(TopkLds*)tkb_lds;
+  const int64_t row = blockIdx.x;
+  {
+    float v[TKB_MAX_BLOCKS / 1024];
+    int32_t id[TKB_MAX_BLOCKS / 1024];
+#pragma unroll
+    for (int j = 0; j < TKB_MAX_BLOCKS / 1024; ++j) {
+      const int64_t c = threadIdx.x + 1024 * j;
+      v[j] = c < C ? best_v[row * C + c] : -INFINITY;
+      id[j] = c < C ? best_i[row * C + c] : INT32_MAX;
+    }
+    topk_pick(L, v, id, k);
+  }
+  float v[2];
+  int32_t id[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int b = (threadIdx.x >> 6) + 16 * j;
+    v[j] = -INFINITY, id[j] = INT32_MAX;
+    if (b < k && L.top_i[b] != INT32_MAX) {
+      const int32_t n = (L.top_i[b] & ~(HD_ROWS - 1)) + (threadIdx.x & 63);
+      const float lv = n < V ? logits[row * ld + n] : -INFINITY;
+      if (n < V && lv == lv) v[j] = lv, id[j] = n;
+    }
+  }
+  __syncthreads();  // the blocks have been read from L.top
+  topk_pick(L, v, id, k);
+  if ((int)threadIdx.x < k) {
+    out_v[row * k + threadIdx.x] = Elem<ODT>::cvt(L.top_v[threadIdx.x]);
+    out_i[row * k + threadIdx.x] = L.top_i[threadIdx.x];
+  }
+}
+
+// What the MFMA form takes: tiles of 4 rows, 16-bit aligned x, whole 128-k blocks within a group.
+template <int XDT>
+bool head_mfma_ok(const void* x, int64_t M, int64_t K, int64_t xs, const void* qw, int64_t T, int64_t gsz) {
+  return XDT != ANNA_MI_F32 && T == 4 && M >= 1 && K % 128 == 0 && gsz % 128 == 0 && xs % 8 == 0 &&
+         (uintptr_t)x % 16 == 0 && (uintptr_t)qw % 16 == 0 && (M + 15) / 16 < 65536;
+}
+
+template <int XDT, int SDT, bool OUT_F32>
+int launch_head_mfma(const void* x, int64_t M, int64_t K, int64_t xs, const uint32_t* qw, int64_t tiles, int64_t pc,
+                     const void* qs, const int8_t* qz, int64_t ssg, int64_t ssn, int64_t gsz, int64_t N, void* y,
+                     int64_t ys, float* best_v, int32_t* best_i, hipStream_t st) {
+  const dim3 grid((unsigned)((N + HD_ROWS - 1) / HD_ROWS), (unsigned)((M + 15) / 16));
+  auto go = [&](auto mp_tag) {
+    constexpr int MP = decltype(mp_tag)::value;
+    auto kern = int4_head_mfma_kernel<XDT, SDT, MP, OUT_F32>;
+    constexpr size_t lds = sizeof(HeadLds<MP>);
+    if constexpr (lds > 65536)
+      ANNA_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess,
+                 "int4 LM head: cannot raise the LDS limit");
+    hipLaunchKernelGGL(kern, grid, dim3(64 * HD_WAVES), lds, st, (const uint16_t*)x, M, K, xs, qw, tiles, pc,
+                       (const typename Elem<SDT>::T*)qs, qz, ssg, ssn, gsz / 128, N, y, ys, best_v, best_i);
+    return ANNA_MI_OK;
+  };
+  const int rc = M <= 1   ? go(std::integral_constant<int, 1>{})
+                 : M <= 2 ? go(std::integral_constant<int, 2>{})
+                 : M <= 4 ? go(std::integral_constant<int, 4>{})
+                 : M <= 8 ? go(std::integral_constant<int, 8>{})
+                          : go(std::integral_constant<int, 16>{});
+  if (rc != ANNA_MI_OK) return rc;
+  ANNA_LAUNCH_CHECK("int4_head_mfma_kernel");
+  return ANNA_MI_OK;
+}
+
 // ANNA_MI_TILED_PLAIN=1 keeps the tiled GEMV off its LDS-staged form (for comparisons and tests)
 static const int g_tiled_plain = [] {
   const char* v = getenv("ANNA_MI_TILED_PLAIN");
@@ -723,6 +1019,13 @@ int launch_tiled(const void* x, int64_t M, int64_t K, int64_t xs, const uint32_t
                  int64_t ys, hipStream_t st) {
   using XT = typename Elem<XDT>::T;
   using ST = typename Elem<SDT>::T;
+  // 40.0 against 42.7 us for one row (V = 151936, K = 2048), 42.5 against 104.9 for four, 92 against
+  // 452 for sixteen
+  if constexpr (XDT != ANNA_MI_F32) {
+    if (head_mfma_ok<XDT>(x, M, K, xs, qw, T, gsz) && !g_tiled_plain)
+      return launch_head_mfma<XDT, SDT, OUT_F32>(x, M, K, xs, qw, tiles, pc, qs, qz, ssg, ssn, gsz, N, y, ys, nullptr,
+                                                 nullptr, st);
+  }
   const dim3 grid((unsigned)((tiles + 3) / 4));
 #define ANNA_TILED_LAUNCH(TT)                                                                                  \
   hipLaunchKernelGGL((int4_gemv_tiled_kernel<XDT, SDT, TT, OUT_F32>), grid, dim3(256), 0, st, (const XT*)x, M, K, \
@@ -860,4 +1163,50 @@ extern "C" int anna_mi_lm_head_int4_topk(const void* x, int x_dtype, int64_t row
                                    vocab, logits, 1, vocab, stream);
   if (rc != ANNA_MI_OK) return rc;
   return topk_rows(logits, rows, vocab, vocab, top_k, values, x_dtype, indices, stream, true);
+}
+
+extern "C" int64_t anna_mi_lm_head_int4_topk_workspace(int64_t rows, int64_t vocab) {
+  return rows * vocab + rows * ((vocab + HD_ROWS - 1) / HD_ROWS) * 2;
+}
+
+extern "C" int anna_mi_lm_head_int4_topk_ws(const void* x, int x_dtype, int64_t rows, int64_t K, int64_t x_row_stride,
+                                            const int32_t* qweight, int64_t tiles, int64_t packed_cols, int64_t tile,
+                                            const void* qscale, int scale_dtype, const int8_t* qzeros,
+                                            int64_t group_count, int64_t scale_stride_group, int64_t scale_stride_row,
+                                            int64_t group_size, int64_t vocab, int64_t top_k, float* workspace,
+                                            void* values, int64_t* indices, void* stream) {
+  ANNA_CHECK(workspace && values && indices, "anna_mi_lm_head_int4_topk: null pointer");
+  const int64_t C = (vocab + HD_ROWS - 1) / HD_ROWS;
+  bool fused = false;
+  ANNA_DISPATCH_DTYPE(x_dtype, XDT, {
+    fused = head_mfma_ok<XDT>(x, rows, K, x_row_stride, qweight, tile, group_size) && !g_tiled_plain;
+  });
+  // (short rows: one workgroup reads them whole)
+  if (!fused || C > TKB_MAX_BLOCKS || vocab < 8192 || vocab >= INT32_MAX || top_k < 1 || top_k > TK_MAX)
+    return anna_mi_lm_head_int4_topk(x, x_dtype, rows, K, x_row_stride, qweight, tiles, packed_cols, tile, qscale,
+                                     scale_dtype, qzeros, group_count, scale_stride_group, scale_stride_row, group_size,
+                                     vocab, top_k, workspace, values, indices, stream);
+  const int rc = check_tiled(x, rows, K, x_row_stride, (const uint32_t*)qweight, tiles, packed_cols, tile, qscale,
+                             qzeros, group_count, group_size, vocab);
+  if (rc != ANNA_MI_OK) return rc;
+  float* const best_v = workspace + rows * vocab;
+  int32_t* const best_i = (int32_t*)(best_v + rows * C);
+  ANNA_DISPATCH_DTYPE(x_dtype, XDT, {
+    if constexpr (XDT != ANNA_MI_F32) {
+      ANNA_DISPATCH_DTYPE(scale_dtype, SDT, {
+        const int rc2 = launch_head_mfma<XDT, SDT, true>(x, rows, K, x_row_stride, (const uint32_t*)qweight, tiles,
+                                                         packed_cols, qscale, qzeros, scale_stride_group,
+                                                         scale_stride_row, group_size, vocab, workspace, vocab, best_v,
+                                                         best_i, as_stream(stream));
+        if (rc2 != ANNA_MI_OK) return rc2;
+      });
+      ANNA_CHECK(hipFuncSetAttribute((const void*)topk_blocks_kernel<XDT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)sizeof(TopkLds)) == hipSuccess,
+                 "int4 LM head: cannot raise the LDS limit");
+      hipLaunchKernelGGL((topk_blocks_kernel<XDT>), dim3((unsigned)rows), dim3(1024), sizeof(TopkLds), as_stream(stream), workspace,
+                         vocab, vocab, best_v, best_i, C, (int)top_k, (typename Elem<XDT>::T*)values, indices);
+    }
+  });
+  ANNA_LAUNCH_CHECK("topk_blocks_kernel");
+  return ANNA_MI_OK;
 }

@@ -887,7 +887,7 @@ __global__ __launch_bounds__(256) void tq_append_kernel(const anna_mi_tq_append_
 // anna_mi_tq_hadamard_quantize) and writes key codes token-major, value codes in the 32-token
 // blocked layout, and the fp16 norms.
 template <int QPW>  // quads of 4 tokens per wave: their vectors go through the transform together
-__global__ __launch_bounds__(256) void tq_pack_kv_kernel(const anna_mi_tq_pack_args a) {
+__device__ __forceinline__ void pack_kv(const anna_mi_tq_pack_args& a) {
   constexpr int NV = 4 * QPW;
   const int lane = threadIdx.x & 63;
   const int64_t groups = (a.tokens + NV - 1) / NV;
@@ -945,6 +945,61 @@ __global__ __launch_bounds__(256) void tq_pack_kv_kernel(const anna_mi_tq_pack_a
       }
     }
     if (lane < nvalid) a.value_norms[h * T + slot0 + lane] = f32_to_f16_bits(nrm_lane);
+  }
+}
+
+template <int QPW>
+__global__ __launch_bounds__(256) void tq_pack_kv_kernel(const anna_mi_tq_pack_args a) {
+  pack_kv<QPW>(a);
+}
+
+// A sequence's whole prefill: the first pack_wgs workgroups quantize, the others copy the newest
+// tokens into the ring -- one wave per (KV head, 8 ring slots): key rows slot by slot, values
+// transposed in registers (a lane holds 4 dims of 8 tokens, whose ring slots are 16 consecutive bytes
+// of a dim's row).  The copies and the length were ten more launches (arange, remainder, two
+// index_puts with their index kernels, a fill).
+__global__ __launch_bounds__(256) void tq_load_kernel(const anna_mi_tq_load_args a, uint32_t pack_wgs) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.seq_length = (int32_t)a.length;
+  if (blockIdx.x < pack_wgs) {
+    pack_kv<1>(a.pack);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int64_t w = (int64_t)(blockIdx.x - pack_wgs) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t R = a.residual_capacity, per = R / 8;
+  if (w >= a.pack.kv_heads * per) return;
+  const int64_t h = w / per, s0 = (w - h * per) * 8;
+  const uint16_t* const ks = a.pack.keys + h * a.pack.stride_head + 4 * lane;
+  const uint16_t* const vs = a.pack.values + h * a.pack.stride_head + 4 * lane;
+  uint16_t v[8][4];
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    // the newest token of ring slot s0 + i, if the sequence has one
+    const int64_t s = s0 + i, last = a.length - 1;
+    const int64_t t = last - ((last - s) % R + R) % R;
+    const bool ok = t >= 0;
+    const uint2 kv = *(const uint2*)(ks + (ok ? t : 0) * a.pack.stride_token);
+    const uint2 vv = *(const uint2*)(vs + (ok ? t : 0) * a.pack.stride_token);
+    any = any || ok;
+    if (ok) *(uint2*)(a.residual_key + (h * R + s) * TD + 4 * lane) = kv;
+    v[i][0] = (uint16_t)(vv.x & 0xFFFFu), v[i][1] = (uint16_t)(vv.x >> 16);
+    v[i][2] = (uint16_t)(vv.y & 0xFFFFu), v[i][3] = (uint16_t)(vv.y >> 16);
+  }
+  if (!any) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    uint16_t* dst = a.residual_value_t + (h * TD + 4 * lane + e) * R + s0;
+    if (s0 + 8 <= a.length) {
+      u32x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = (uint32_t)v[2 * i][e] | ((uint32_t)v[2 * i + 1][e] << 16);
+      *(u32x4*)dst = o;
+    } else {  // slots past a sequence shorter than the window are left as they are
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (s0 + i < a.length) dst[i] = v[i][e];
+    }
   }
 }
 
@@ -1076,26 +1131,57 @@ extern "C" int anna_mi_tq_append(const anna_mi_tq_append_args* ap, void* stream)
 
 extern "C" int64_t anna_mi_sizeof_tq_pack_args(void) { return (int64_t)sizeof(anna_mi_tq_pack_args); }
 
+namespace anna {
+namespace {
+int check_pack(const anna_mi_tq_pack_args& a, const char* what) {
+  ANNA_CHECK(a.head_dim == TD, "%s: head_dim must be 256", what);
+  ANNA_CHECK(a.keys && a.values && a.key_codes && a.key_norms && a.value_codes && a.value_norms && a.signs &&
+                 a.thresholds,
+             "%s: null pointer", what);
+  ANNA_CHECK(a.kv_heads > 0 && a.tokens >= 0, "%s: bad sizes", what);
+  ANNA_CHECK(a.slot_offset % TBT == 0 && a.pool_tokens % TBT == 0 && a.slot_offset + a.tokens <= a.pool_tokens,
+             "%s: slots must start at a multiple of 32 and fit the pool", what);
+  ANNA_CHECK(a.stride_token >= TD && a.stride_token % 4 == 0 && a.stride_head % 4 == 0 &&
+                 (uintptr_t)a.keys % 8 == 0 && (uintptr_t)a.values % 8 == 0,
+             "%s: rows must be 8-byte aligned with a stride of at least 256", what);
+  return ANNA_MI_OK;
+}
+// one quad per wave: the kernel is VALU-bound (about 600 VALU instructions per wave at 8 waves per
+// SIMD), and two quads per wave measured slower (fewer waves to hide the exchanges)
+constexpr int PACK_QPW = 1;
+int64_t pack_workgroups(const anna_mi_tq_pack_args& a) {
+  const int64_t waves = 2 * a.kv_heads * ((a.tokens + 4 * PACK_QPW - 1) / (4 * PACK_QPW));
+  return (waves + 3) / 4;
+}
+}  // namespace
+}  // namespace anna
+
 extern "C" int anna_mi_tq_pack_kv(const anna_mi_tq_pack_args* ap, void* stream) {
   ANNA_CHECK(ap != nullptr, "anna_mi_tq_pack_kv: null args");
   const anna_mi_tq_pack_args& a = *ap;
-  ANNA_CHECK(a.head_dim == TD, "anna_mi_tq_pack_kv: head_dim must be 256");
-  ANNA_CHECK(a.keys && a.values && a.key_codes && a.key_norms && a.value_codes && a.value_norms && a.signs &&
-                 a.thresholds,
-             "anna_mi_tq_pack_kv: null pointer");
-  ANNA_CHECK(a.kv_heads > 0 && a.tokens >= 0, "anna_mi_tq_pack_kv: bad sizes");
-  ANNA_CHECK(a.slot_offset % TBT == 0 && a.pool_tokens % TBT == 0 && a.slot_offset + a.tokens <= a.pool_tokens,
-             "anna_mi_tq_pack_kv: slots must start at a multiple of 32 and fit the pool");
-  ANNA_CHECK(a.stride_token >= TD && a.stride_token % 4 == 0 && a.stride_head % 4 == 0 &&
-                 (uintptr_t)a.keys % 8 == 0 && (uintptr_t)a.values % 8 == 0,
-             "anna_mi_tq_pack_kv: rows must be 8-byte aligned with a stride of at least 256");
+  if (const int rc = check_pack(a, "anna_mi_tq_pack_kv"); rc != ANNA_MI_OK) return rc;
   if (a.tokens == 0) return ANNA_MI_OK;
-  // one quad per wave: the kernel is VALU-bound (about 600 VALU instructions per wave at 8
-  // waves per SIMD), and two quads per wave measured slower (fewer waves to hide the exchanges)
-  constexpr int QPW = 1;
-  const int64_t waves = 2 * a.kv_heads * ((a.tokens + 4 * QPW - 1) / (4 * QPW));
-  hipLaunchKernelGGL(tq_pack_kv_kernel<QPW>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, as_stream(stream), a);
+  hipLaunchKernelGGL(tq_pack_kv_kernel<PACK_QPW>, dim3((unsigned)pack_workgroups(a)), dim3(256), 0, as_stream(stream), a);
   ANNA_LAUNCH_CHECK("tq_pack_kv_kernel");
+  return ANNA_MI_OK;
+}
+
+extern "C" int64_t anna_mi_sizeof_tq_load_args(void) { return (int64_t)sizeof(anna_mi_tq_load_args); }
+
+extern "C" int anna_mi_tq_load(const anna_mi_tq_load_args* ap, void* stream) {
+  ANNA_CHECK(ap != nullptr, "anna_mi_tq_load: null args");
+  const anna_mi_tq_load_args& a = *ap;
+  if (const int rc = check_pack(a.pack, "anna_mi_tq_load"); rc != ANNA_MI_OK) return rc;
+  const int64_t R = a.residual_capacity;
+  ANNA_CHECK(R > 0 && R % 32 == 0, "anna_mi_tq_load: the window must be a multiple of 32 tokens");
+  ANNA_CHECK(a.length > 0 && a.length < (1ll << 31) && a.pack.tokens <= a.length, "anna_mi_tq_load: bad length");
+  ANNA_CHECK(a.residual_key && a.residual_value_t && a.seq_length, "anna_mi_tq_load: null pointer");
+  ANNA_CHECK((uintptr_t)a.residual_key % 16 == 0 && (uintptr_t)a.residual_value_t % 16 == 0,
+             "anna_mi_tq_load: the rings must be 16-byte aligned");
+  const int64_t pack_wgs = pack_workgroups(a.pack), ring_wgs = (a.pack.kv_heads * (R / 8) + 3) / 4;
+  hipLaunchKernelGGL(tq_load_kernel, dim3((unsigned)(pack_wgs + ring_wgs)), dim3(256), 0, as_stream(stream), a,
+                     (uint32_t)pack_wgs);
+  ANNA_LAUNCH_CHECK("tq_load_kernel");
   return ANNA_MI_OK;
 }
 

@@ -683,12 +683,13 @@ def lm_head_int4_topk(hidden_states, qweight, qscale, qzeros, group_size, in_fea
     if x.stride(1) != 1:
         x = x.contiguous()
     rows = x.shape[0]
-    logits = torch.empty((rows, vocab), dtype=torch.float32, device=x.device)
+    words = _lib.load().anna_mi_lm_head_int4_topk_workspace(rows, vocab)  # logits, then each block's best
+    workspace = torch.empty((words,), dtype=torch.float32, device=x.device)
     values = torch.empty((rows, top_k), dtype=x.dtype, device=x.device)
     indices = torch.empty((rows, top_k), dtype=torch.int64, device=x.device)
-    _lib.call("anna_mi_lm_head_int4_topk", x.data_ptr(), _lib.dtype_code(x.dtype), rows, in_features, x.stride(0),
+    _lib.call("anna_mi_lm_head_int4_topk_ws", x.data_ptr(), _lib.dtype_code(x.dtype), rows, in_features, x.stride(0),
               qweight.data_ptr(), tiles, pc, tile, qscale.data_ptr(), _lib.dtype_code(qscale.dtype), qzeros.data_ptr(),
-              g, ssg, ssn, int(group_size), vocab, int(top_k), logits.data_ptr(), values.data_ptr(), indices.data_ptr(),
+              g, ssg, ssn, int(group_size), vocab, int(top_k), workspace.data_ptr(), values.data_ptr(), indices.data_ptr(),
               _lib.stream_of(x))
     return values.view(*lead, top_k), indices.view(*lead, top_k)
 

@@ -112,20 +112,42 @@ class TurboQuantBatchCache:
         q = max(0, L - R)
         if q > self.capacities[b]:
             raise ValueError(f"sequence {b}: {q} quantized tokens exceed its capacity {self.capacities[b]}")
-        off = self.offsets[b]
-        if q > 0:
-            if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
-                raise ValueError("keys/values must be bf16")
-            k, v = keys, values
-            if k.stride(2) != 1 or v.stride() != k.stride():  # the pack reads both with one set of strides
-                k, v = keys.contiguous(), values.contiguous()
-            self._pack(k, v, q, off)
-        if L > q:
-            slots = torch.arange(q, L, device=self.device) % R
-            self.residual_key[b][:, slots] = keys[:, q:]
-            self.residual_value_t[b][:, :, slots] = values[:, q:].transpose(1, 2)
-        self.seq_lengths[b] = L
+        if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
+            raise ValueError("keys/values must be bf16")
+        if D != self.head_dim:
+            raise ValueError(f"keys/values must have head_dim {self.head_dim}, got {D}")
+        if L == 0:
+            self.seq_lengths[b] = 0
+        else:
+            k, v = keys.expand(self.kv_heads, L, D), values.expand(self.kv_heads, L, D)
+            self._load(range(self.batch)[b], k, v, q)
         self.lengths[b] = L
+
+    def _load(self, b: int, keys: torch.Tensor, values: torch.Tensor, tokens: int) -> None:
+        """One launch: the first `tokens` tokens of keys/values [Hkv, L, D] into the pool, the newest
+        ones into the ring, and the length."""
+        _lib.require_device(keys, values, self.residual_key)
+        # the launch reads both with one set of strides, 8 bytes of a row at a time
+        if (keys.stride(2) != 1 or values.stride() != keys.stride() or keys.stride(0) % 4 or keys.stride(1) % 4
+                or keys.stride(1) < keys.shape[2] or keys.data_ptr() % 8 or values.data_ptr() % 8):
+            keys, values = (t.contiguous() if t.data_ptr() % 8 == 0 else t.clone(memory_format=torch.contiguous_format)
+                            for t in (keys, values))
+        a = _lib.TQLoadArgs()
+        p = a.pack
+        p.kv_heads, p.head_dim, p.tokens = self.kv_heads, self.head_dim, tokens
+        p.keys, p.values = keys.data_ptr(), values.data_ptr()
+        p.stride_head = keys.stride(0) if self.kv_heads > 1 else 0
+        p.stride_token = max(keys.stride(1), self.head_dim)
+        p.key_codes, p.key_norms = self.key_codes.data_ptr(), self.key_norms.data_ptr()
+        p.value_codes, p.value_norms = self.value_codes.data_ptr(), self.value_norms.data_ptr()
+        p.pool_tokens, p.slot_offset = self.pool_tokens, self.offsets[b]
+        p.signs, p.thresholds = self.qn.signs.data_ptr(), self.qn.thresholds.data_ptr()
+        H, R, D = self.kv_heads, self.residual_capacity, self.head_dim
+        a.length, a.residual_capacity = keys.shape[1], R
+        a.residual_key = self.residual_key.data_ptr() + 2 * b * H * R * D
+        a.residual_value_t = self.residual_value_t.data_ptr() + 2 * b * H * R * D
+        a.seq_length = self.seq_lengths.data_ptr() + 4 * b
+        _lib.call("anna_mi_tq_load", ctypes.byref(a), _lib.stream_of(keys))
 
     def _pack(self, keys: torch.Tensor, values: torch.Tensor, tokens: int, slot_offset: int) -> None:
         """One launch: the first `tokens` tokens of keys/values [Hkv, L, D] into the pool."""

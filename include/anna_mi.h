@@ -465,6 +465,21 @@ typedef struct {
  * counterpart of the per-token quantization in TurboQuantKVRow.append (turboquant.py:1027-1140)
  * and of TurboQuantTensorRow.append (turboquant.py:335-477) for BASELINE config 3. */
 int anna_mi_tq_pack_kv(const anna_mi_tq_pack_args* args, void* stream);
+
+/* anna_mi_tq_pack_kv (skipped when pack.tokens is 0) plus the rest of a sequence's prefill in the same
+ * launch: the newest min(length, R) of its `length` tokens into the window ring (token j at slot
+ * j % R) and the length itself.  pack.keys / pack.values hold the whole history (pack.tokens of it
+ * are quantized). */
+typedef struct {
+  anna_mi_tq_pack_args pack;
+  int64_t length;
+  uint16_t* residual_key;     /* the sequence's ring: bf16 [Hkv, R, 256] */
+  uint16_t* residual_value_t; /* bf16 [Hkv, 256, R] */
+  int64_t residual_capacity;  /* R, a multiple of 32 */
+  int32_t* seq_length;        /* device: the sequence's length */
+} anna_mi_tq_load_args;
+int anna_mi_tq_load(const anna_mi_tq_load_args* args, void* stream);
+int64_t anna_mi_sizeof_tq_load_args(void);
 int64_t anna_mi_sizeof_tq_pack_args(void);
 
 /* Reorders natural 2-bit codes [tokens][64] (D = 256) of one KV head into the blocked value
@@ -503,6 +518,17 @@ int anna_mi_lm_head_int4_topk(const void* x, int x_dtype, int64_t rows, int64_t 
                               const void* qscale, int scale_dtype, const int8_t* qzeros, int64_t group_count,
                               int64_t scale_stride_group, int64_t scale_stride_row, int64_t group_size, int64_t vocab,
                               int64_t top_k, float* logits, void* values, int64_t* indices, void* stream);
+
+/* The same with room for per-block bests beside the logits: workspace holds
+ * anna_mi_lm_head_int4_topk_workspace(rows, vocab) floats (the logits first).  16-bit x with whole
+ * 128-k blocks on tiles of 4 then takes one GEMV and one selection over 64-logit blocks. */
+int64_t anna_mi_lm_head_int4_topk_workspace(int64_t rows, int64_t vocab);
+int anna_mi_lm_head_int4_topk_ws(const void* x, int x_dtype, int64_t rows, int64_t K, int64_t x_row_stride,
+                                 const int32_t* qweight, int64_t tiles, int64_t packed_cols, int64_t tile,
+                                 const void* qscale, int scale_dtype, const int8_t* qzeros, int64_t group_count,
+                                 int64_t scale_stride_group, int64_t scale_stride_row, int64_t group_size,
+                                 int64_t vocab, int64_t top_k, float* workspace, void* values, int64_t* indices,
+                                 void* stream);
 
 /* ------------------------------------------------------------------ MoE
  * Routing around the grouped expert MLP (Qwen3SparseMoeBlock, src/anna/model/ops.py:3280-3376). */

@@ -144,3 +144,44 @@ def test_lm_head_topk_exact_ties_in_wave_path(gpu, layout):
         assert indices[r].cpu().tolist() == order
         got = values[r].float().cpu()
         assert torch.equal(got[0::2], got[1::2])  # twins carry the same value
+
+
+@pytest.mark.parametrize("k,n,rows,top_k,dtype,group", [
+    (128, 8192, 1, 1, torch.bfloat16, 128), (256, 8196, 2, 8, torch.float16, 128), (512, 9000, 3, 32, torch.bfloat16, 128),
+    (640, 16444, 5, 20, torch.float16, 128), (1024, 70004, 9, 8, torch.bfloat16, 256),
+    (2048, 12300, 17, 9, torch.bfloat16, 128), (2176, 8260, 33, 5, torch.float16, 128),
+])
+def test_lm_head_block_selection(gpu, k, n, rows, top_k, dtype, group):
+    """Whole 128-k blocks on tiles of 4 rows: the MFMA GEMV (K short of four waves' shares, ragged last
+    block of rows, one to three 16-row blocks of x) and the selection over 64-logit blocks, against fp64;
+    repeated weight rows make exact ties, which go to the lower index."""
+    torch.manual_seed(k + n)
+    kp = -(-k // group) * group
+    q = XPUInt4Linear(k, n, group_size=group, compute_dtype=dtype, device=gpu)
+    with torch.no_grad():
+        q.qweight.copy_(torch.randint(-(2**31), 2**31, (n, kp // 8), dtype=torch.int32, device=gpu))
+        q.qscale.copy_(torch.rand(kp // group, n, device=gpu) * 0.01 + 0.001)
+        q.qzeros.copy_(torch.randint(-128, 128, (kp // group, n), dtype=torch.int8, device=gpu))
+        for buf, dim in ((q.qweight, 0), (q.qscale, 1), (q.qzeros, 1)):  # the last 70 rows repeat the first 70
+            buf.narrow(dim, n - 70, 70).copy_(buf.narrow(dim, 0, 70))
+    q.prepare_lm_head_topk_layout()
+    x = torch.randn(rows, k, device=gpu, dtype=dtype)
+    values, indices = torch.ops.anna.lm_head_int4_topk_fused(x, q.lm_head_qweight, q.lm_head_qscale, q.lm_head_qzeros,
+                                                             group, k, top_k)
+    ref = dense_logits(q, x).to(gpu)
+    rv, _ = torch.topk(ref, top_k, dim=-1)
+    # fp32 sums of up to 2176 products of |code - zero| <= 143 against values of a few hundred, then the
+    # output's rounding (2^-9 or 2^-12 of the value)
+    eps = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-10
+    scale = ref.abs().amax()
+    assert ((values.double() - rv).abs() <= eps * rv.abs() + 1e-5 * scale).all()
+    assert ((torch.gather(ref, 1, indices) - rv).abs() <= 1e-5 * scale).all()
+    assert all(len(set(r.tolist())) == top_k for r in indices)
+    for row in indices.tolist():  # a repeated row never stands before the row it repeats
+        for place, i in enumerate(row):
+            if i >= n - 70:
+                assert i - (n - 70) in row[:place]
+    # the GEMV alone, in the activation dtype
+    y = fused_ops.int4_gemv_tiled(x, q.lm_head_qweight, q.qscale.view(-1, n // 4, 4), q.qzeros.view(-1, n // 4, 4),
+                                  group, k, n)
+    assert rel_err(y.double().cpu().numpy(), ref.cpu().numpy()) <= BF16_TOL

@@ -130,3 +130,33 @@ def test_store_refusals(gpu):
     other.update(odd, odd, 0, require_dense_cache=False)
     with pytest.raises(ValueError):
         other.update(odd, odd, 0, require_dense_cache=False)
+
+
+@pytest.mark.parametrize("length", [1, 31, 64, 65, 190, 417])
+@pytest.mark.parametrize("window", [32, 64])
+def test_pool_load_equals_appends(gpu, length, window):
+    """load_sequence of the 2-bit pool over a row that held other tokens leaves what as many appends
+    leave, for separate and interleaved layouts of keys and values."""
+    torch.manual_seed(length)
+    batch, heads, D = 2, 3, 256
+    caches = [TurboQuantBatchCache(batch=batch, kv_heads=heads, q_heads=2 * heads, capacities=[448, 450],
+                                   residual_capacity=window) for _ in range(2)]
+    k, v = (torch.randn(length, batch, heads, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+    for t in range(length):
+        caches[0].append(k[t], v[t])
+    caches[1].load_sequence(0, *(torch.randn(heads, 300, D, device=gpu, dtype=torch.bfloat16) for _ in range(2)))
+    caches[1].load_sequence(0, k[:, 0].transpose(0, 1), v[:, 0].transpose(0, 1).contiguous())
+    caches[1].load_sequence(1, k[:, 1].transpose(0, 1), v[:, 1].transpose(0, 1))
+    one, two = caches
+    assert one.lengths == two.lengths == one.seq_lengths.tolist() == two.seq_lengths.tolist()
+    q, r = max(0, length - window), min(length, window)
+    for b in range(batch):
+        s = slice(one.offsets[b], one.offsets[b] + q)
+        for name in ("key_codes", "key_norms", "value_norms"):
+            same(getattr(one, name)[:, s], getattr(two, name)[:, s])
+        whole = slice(one.offsets[b] // 32, (one.offsets[b] + q // 32 * 32) // 32)  # blocks of 32 slots
+        same(one.value_codes[:, whole], two.value_codes[:, whole])
+    same(one.residual_key[:, :, :r], two.residual_key[:, :, :r])
+    same(one.residual_value_t[..., :r], two.residual_value_t[..., :r])
+    query = torch.randn(batch, 2 * heads, D, device=gpu, dtype=torch.bfloat16)
+    same(one.decode(query, scaling=0.06), two.decode(query, scaling=0.06))
