@@ -556,8 +556,9 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(const anna_
 // the four sums are added in wave order, so the result does not depend on timing.
 constexpr int MERGE_DIM_WAVES = 4;
 constexpr int MERGE_DIM_MAXBLK = 64 * MERGE_DIM_WAVES;
-constexpr int MERGE_DIM_PRE = 32;  // partial values per lane loaded before the reductions
-
+// PRE: partial values per lane loaded before the reductions -- a wave's whole share, 32 up to 128
+// blocks and 64 above (254 blocks with 32: 18.7 us, the rest of the share read in rounds of 8).
+template <int MERGE_DIM_PRE>
 __global__ __launch_bounds__(64 * MERGE_DIM_WAVES) void decode_merge_dims_kernel(const anna_mi_decode_args a,
                                                                                  int64_t nblk) {
   __shared__ float s_w[MERGE_DIM_MAXBLK];
@@ -605,12 +606,6 @@ __global__ __launch_bounds__(64 * MERGE_DIM_WAVES) void decode_merge_dims_kernel
       const float w = s_w[k0 + i];
       if (w != 0.f) acc += w * pre[i];
     }
-  }
-#pragma unroll 8
-  for (int k = k0 + MERGE_DIM_PRE; k < k1; ++k) {
-    const float v = vd[(int64_t)k * pv.s2];
-    const float w = s_w[k];
-    if (w != 0.f) acc += w * v;
   }
   s_sum[wave][lane] = acc;
   __syncthreads();
@@ -1578,8 +1573,11 @@ static int gqa_decode_splitkv_impl(const anna_mi_decode_args& a, void* stream) {
   ANNA_LAUNCH_CHECK("decode_split_kernel");
   const int64_t nrot = a.value_format == ANNA_MI_VALUES_TQ_MSE ? sp.nb1 : 0;
   if (nrot == 0 && nmerge <= MERGE_DIM_MAXBLK) {
-    hipLaunchKernelGGL(decode_merge_dims_kernel, dim3((unsigned)(a.head_dim / 64), (unsigned)a.q_heads, (unsigned)a.batch),
-                       dim3(64 * MERGE_DIM_WAVES), 0, st, a, nmerge);
+    const dim3 grid((unsigned)(a.head_dim / 64), (unsigned)a.q_heads, (unsigned)a.batch);
+    if (nmerge <= 32 * MERGE_DIM_WAVES)
+      hipLaunchKernelGGL(decode_merge_dims_kernel<32>, grid, dim3(64 * MERGE_DIM_WAVES), 0, st, a, nmerge);
+    else
+      hipLaunchKernelGGL(decode_merge_dims_kernel<64>, grid, dim3(64 * MERGE_DIM_WAVES), 0, st, a, nmerge);
     ANNA_LAUNCH_CHECK("decode_merge_dims_kernel");
   } else {
     hipLaunchKernelGGL(decode_merge_kernel, dim3((unsigned)a.q_heads, (unsigned)a.batch), dim3(MERGE_THREADS),
