@@ -9,6 +9,7 @@ is raised.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import threading
 from pathlib import Path
 
@@ -250,6 +251,35 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+_HOST_ENTRIES = ("anna_mi_last_error", "anna_mi_int4_linear", "anna_mi_decode_num_blocks", "anna_mi_gqa_decode_splitkv",
+                 "anna_mi_tq_decode", "anna_mi_tq_store", "anna_mi_moe_route_small", "anna_mi_moe_gather",
+                 "anna_mi_moe_router", "anna_mi_moe_dispatch", "anna_mi_moe_grouped_int4_mlp", "anna_mi_moe_combine")
+_host = None
+
+
+def host():
+    """The host module (csrc/torch_host.cpp), bound to the library.  Its functions answer None to
+    calls they leave to their Python callers."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is None:
+            path = LIB_PATH.parent / "_torch_host.so"
+            if not path.exists():
+                raise RuntimeError(f"anna_mi host module not built ({path} missing); run `python -m anna_amd.build`")
+            spec = importlib.util.spec_from_file_location("_torch_host", path)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            if module.source_hash() != lib.anna_mi_source_hash().decode():
+                raise RuntimeError(f"{path.name} is stale: it and {LIB_PATH.name} were built from different sources; "
+                                   "run `python -m anna_amd.build`")
+            module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_ENTRIES})
+            _host = module
+    return _host
+
+
 def call(name: str, *args) -> None:
     lib = load()
     rc = getattr(lib, name)(*args)
@@ -278,7 +308,7 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def require_device(*tensors: torch.Tensor) -> None:

@@ -13,12 +13,15 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 OBJ_DIR = PKG_DIR / "_build"
 LIB_PATH = PKG_DIR / "libanna_mi.so"
+HOST_SRC = CSRC / "torch_host.cpp"  # the calls' host side on torch's C++ tensors: its own module
+HOST_PATH = PKG_DIR / "_torch_host.so"
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -45,7 +48,7 @@ def _hipcc() -> str:
 
 
 def _sources() -> list[Path]:
-    return sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.cpp"))
+    return sorted(CSRC.glob("*.hip")) + sorted(p for p in CSRC.glob("*.cpp") if p != HOST_SRC)
 
 
 def source_hash() -> str:
@@ -92,6 +95,23 @@ def _compile(src: Path, stamp: str, force: bool = True) -> Path:
     return obj
 
 
+def _build_host(stamp: str) -> None:
+    """The host module: plain C++ against torch's headers (no device code)."""
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = Path(torch.__file__).resolve().parent / "lib"
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DANNA_MI_SOURCE_HASH="{stamp}"',
+           *(f"-I{p}" for p in cpp_extension.include_paths()), f"-I{sysconfig.get_path('include')}",
+           str(HOST_SRC), "-o", str(tmp), f"-L{torch_lib}", "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for {HOST_SRC.name}:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose: bool = True, force: bool = True) -> Path:
     """Compiles every source (force=False reuses objects newer than their sources and the
     shared headers; the stamped runtime.cpp is always rebuilt) and links the library."""
@@ -100,7 +120,9 @@ def build(verbose: bool = True, force: bool = True) -> Path:
     workers = min(len(sources), max(1, min(8, os.cpu_count() or 1)))
     with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as ex:
         stamp = source_hash()
+        host = ex.submit(_build_host, stamp)
         objs = list(ex.map(lambda src: _compile(src, stamp, force), sources))
+        host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     proc = subprocess.run(cmd, capture_output=True, text=True)

@@ -128,6 +128,11 @@ def int4_linear_out(hidden_states, qweight, qscale, qzeros, group_size, in_featu
 
 
 def _xpu_int4_gemv_impl(hidden_states, qweight, qscale, qzeros, group_size, in_features):
+    if hidden_states.dim() == 2 and hidden_states.size(1) == in_features and qweight.dim() == 2:
+        out = _lib.host().int4_linear(hidden_states, qweight, qscale, qzeros, None, group_size, qweight.size(0),
+                                      hidden_states.dtype, _lib.stream_of(hidden_states), False)
+        if out is not None:
+            return out
     out = torch.empty((hidden_states.size(0), qweight.size(0)), dtype=hidden_states.dtype, device=hidden_states.device)
     return int4_linear_out(hidden_states, qweight, qscale, qzeros, group_size, in_features, out)
 

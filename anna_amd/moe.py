@@ -14,6 +14,7 @@ from dataclasses import dataclass, field
 
 import torch
 
+from . import _lib
 from . import fused_ops
 from .quantization import XPUInt4Linear
 
@@ -83,10 +84,19 @@ class SparseMoeInt4:
     def forward(self, hidden_states: torch.Tensor, router_logits: torch.Tensor) -> torch.Tensor:
         """hidden_states [T, H], router_logits [T, E] -> routed expert output [T, H] (hidden dtype)."""
         t = hidden_states.shape[0]
+        small = t * self.top_k <= 128 and self.num_experts <= 512 and self.top_k <= 64
+        # Routes per expert are only known on the device; the kernels sweep an expert's routes in
+        # as many passes as it needs, so this hint (twice the mean load) only sizes the sweep.
+        hint = max(1, min(t * self.top_k, 2 * -(-t * self.top_k // self.num_experts) + 8))
+        if hidden_states.is_cuda and router_logits.dim() == 2 and router_logits.shape[1] == self.num_experts:
+            out = _lib.host().moe_block(hidden_states, router_logits, *self.bank.tensors(), self.active_experts,
+                                        self.active_slots, self.bank.group_size, self.top_k, self.norm_topk_prob, small,
+                                        hint, _lib.stream_of(hidden_states))
+            if out is not None:
+                return out
         # decode-sized batches: router + dispatch order + the MLP's list of experts with routes in
         # one launch (its single workgroup ranks each route against the earlier ones, which pays
         # only while the routes are few)
-        small = t * self.top_k <= 128 and self.num_experts <= 512 and self.top_k <= 64
         if small:
             w, sel, usage, offsets, _, sri, route_pos, items = fused_ops.moe_route_small(
                 router_logits, self.top_k, self.norm_topk_prob, self.active_slots)
@@ -99,11 +109,8 @@ class SparseMoeInt4:
             _, offsets, compact, cw = fused_ops.moe_dispatch(hidden_states, w, sel, usage, route_pos=route_pos,
                                                               slots=self.active_slots, items=items)
         compact_out = torch.empty_like(compact)
-        # Routes per expert are only known on the device; the kernels sweep an expert's routes in
-        # as many passes as it needs, so this hint (twice the mean load) only sizes the sweep.
-        hint = min(t * self.top_k, 2 * -(-t * self.top_k // self.num_experts) + 8)
         fused_ops.moe_grouped_int4_mlp_out(compact, cw, compact_out, offsets, self.active_experts, self.active_slots,
-                                           *self.bank.tensors(), self.bank.group_size, max(1, hint), items=items,
+                                           *self.bank.tensors(), self.bank.group_size, hint, items=items,
                                            items_prefilled=True)
         return fused_ops.moe_combine(compact_out, route_pos, t, self.top_k)
 

@@ -27,6 +27,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import _lib
 from . import fused_ops
 
 _INT4_PER_WORD = 8
@@ -376,6 +377,12 @@ class XPUInt4Linear(nn.Module):
         return F.linear(x2d, w, bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if x.is_cuda:
+            b, p = self._buffers, self._parameters
+            out = _lib.host().int4_linear(x, b["qweight"], b["qscale"], b["qzeros"], p["bias"], self.group_size,
+                                          self.out_features, self.compute_dtype, _lib.stream_of(x))
+            if out is not None:
+                return out
         lead = x.shape[:-1]
         x2d = x.reshape(-1, x.shape[-1]).to(self.compute_dtype)
         _require_rocm(x2d, "XPUInt4Linear.forward")

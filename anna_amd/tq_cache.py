@@ -228,6 +228,15 @@ class TurboQuantBatchCache:
                gate: torch.Tensor | None = None) -> torch.Tensor:
         """query bf16 [B, Hq, D] -> attention output bf16 [B, Hq, D]; gate (optional, bf16, same
         shape as query): out *= sigmoid(gate) (the reference's gated decode, sycl:1605-1669)."""
+        if query.is_cuda:
+            got = _lib.host().decode_pool(
+                query, gate, out, self.key_codes, self.key_norms, self.value_codes, self.value_norms, self.residual_key,
+                self.residual_value_t, self.seq_offsets, self.seq_lengths, self.qn.signs, self.partial_stats,
+                self.partial_values, self.item_table, self.pool_tokens, self.residual_capacity, self.kv_heads,
+                self.q_heads, self.batch, self.tokens_per_item // 32, self.num_workgroups, self.key_scale,
+                self.value_scale, scaling, _lib.stream_of(query))
+            if got is not None:
+                return got
         query = self._check_query(query, gate)
         gate = None if gate is None else gate.contiguous()
         if out is None:
@@ -378,17 +387,6 @@ class TurboQuantRowsCache(TurboQuantBatchCache):
                gate: torch.Tensor | None = None) -> torch.Tensor:
         """query bf16 [B, Hq, D] -> attention output bf16 [B, Hq, D]; gate (optional, same shape):
         out *= sigmoid(gate)."""
-        shape = (self.batch, self.q_heads, self.head_dim)
-        if query.dtype != torch.bfloat16 or tuple(query.shape) != shape:
-            raise ValueError(f"query must be bf16 [batch, q_heads, {self.head_dim}]")
-        if gate is not None and (gate.dtype != torch.bfloat16 or tuple(gate.shape) != shape):
-            raise ValueError(f"gate must be bf16 [batch, q_heads, {self.head_dim}] (the query's shape)")
-        _lib.require_device(query, gate)
-        q4 = query.contiguous().unsqueeze(2)
-        if out is None:
-            out = torch.empty_like(query)
-        o4 = out.unsqueeze(2)
-        qn = self.qn
         # Blocks sized so that the call is ~1024 workgroups (about four per CU) on the VALU split
         # kernel (other head dims): one per block, KV head and sequence, each writing G partial
         # rows the merge reads back (64-token blocks at 16K tokens made ~4000 workgroups whose
@@ -400,6 +398,25 @@ class TurboQuantRowsCache(TurboQuantBatchCache):
         per_row = max(1, wg // (self.batch * self.kv_heads))
         bs = max(self.block_size, -(-(self.capacity + self.residual_capacity) // per_row))
         bs = -(-bs // 16) * 16
+        qn = self.qn
+        if query.is_cuda and query.dim() == 3 and query.is_contiguous() and (gate is None or gate.is_contiguous()):
+            got = _lib.host().decode_rows(
+                query, gate, out, self.key_codes, self.key_norms, self.value_data, self.value_scales, self.value_zeros,
+                self.residual_key, self.residual_value, self.seq_lengths, qn.rotation, qn.rotation_t, qn.centroids,
+                qn.signs, self.query_rot, self.partial_stats, self.partial_values, self.bits, self.value_group_size,
+                scaling, bs, True, _lib.stream_of(query))
+            if got is not None:
+                return got
+        shape = (self.batch, self.q_heads, self.head_dim)
+        if query.dtype != torch.bfloat16 or tuple(query.shape) != shape:
+            raise ValueError(f"query must be bf16 [batch, q_heads, {self.head_dim}]")
+        if gate is not None and (gate.dtype != torch.bfloat16 or tuple(gate.shape) != shape):
+            raise ValueError(f"gate must be bf16 [batch, q_heads, {self.head_dim}] (the query's shape)")
+        _lib.require_device(query, gate)
+        q4 = query.contiguous().unsqueeze(2)
+        if out is None:
+            out = torch.empty_like(query)
+        o4 = out.unsqueeze(2)
         args = fused_ops.decode_args(
             query=q4, len1=self.capacity, key=self.key_codes, key_format=fused_ops.KEYS_TQ_MSE,
             key_norms=self.key_norms, key_bits=self.bits, value=self.value_data,

@@ -26,8 +26,6 @@ depend on token order, and while a sequence is shorter than the window its token
 
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _lib
@@ -177,34 +175,16 @@ class _LayerSlab:
         _lib.require_device(keys, values, self.rk)
         keys, values = fused_ops.tq_store_rows(keys), fused_ops.tq_store_rows(values)
         qn, ip, C = self._qn, self.key_quantizer == "ip", self.capacity
-        past = torch.empty((self.batch,), dtype=torch.int64, device=self.device)
-        a = _lib.TQStoreArgs()
-        a.dtype, a.key_format = _lib.dtype_code(self.dtype), int(ip)
-        a.batch, a.row0, a.rows = self.batch, row0, rows
-        a.kv_heads, a.head_dim, a.tokens, a.capacity, a.residual_capacity = H, D, T, C, R
-        a.key_bits = a.value_bits = self.bits
-        a.value_group_size = self.value_group_size
-        a.new_key, a.new_value = keys.data_ptr(), values.data_ptr()
-        a.key_stride_row, a.key_stride_head, a.key_stride_token, _ = keys.stride()
-        a.value_stride_row, a.value_stride_head, a.value_stride_token, _ = values.stride()
-        if C > 0:
-            a.key_norms = self.knorms.data_ptr()
-            a.value_data, a.value_scales, a.value_zeros = (self.vdata.data_ptr(), self.vscales.data_ptr(),
-                                                           self.vzeros.data_ptr())
-            if ip:
-                a.key_codes, a.key_signs = self.kidx.data_ptr(), self.kqjl.data_ptr()
-                a.key_residual_norms, a.key_dense = self.krn.data_ptr(), self.kdense.data_ptr()
-            else:
-                a.key_codes = self.kcodes.data_ptr()
-        a.residual_key, a.residual_value = self.rk.data_ptr(), self.rv.data_ptr()
-        a.seq_in, a.seq_out, a.past_out = self.seq_lengths.data_ptr(), self._next_lengths.data_ptr(), past.data_ptr()
-        a.max_leaving = max(max(0, n + T - R) - max(0, n - R) for n in lens)
-        a.max_fill = max(max(0, min(R, n + T) - n) for n in lens)
-        a.signs, a.thresholds = qn.signs.data_ptr(), qn.thresholds.data_ptr()
-        if ip:
-            a.centroids, a.gaussian, a.gaussian_t = (qn.centroids.data_ptr(), qn.gaussian.data_ptr(),
-                                                     qn.gaussian_t.data_ptr())
-        _lib.call("anna_mi_tq_store", ctypes.byref(a), _lib.stream_of(keys))
+        leaving = max(max(0, n + T - R) - max(0, n - R) for n in lens)
+        fill = max(max(0, min(R, n + T) - n) for n in lens)
+        key_state = (None,) * 5 if C == 0 else (
+            (self.kidx, self.knorms, self.kqjl, self.krn, self.kdense) if ip else (self.kcodes, self.knorms, None, None, None))
+        past = _lib.host().tq_store(
+            keys, values, *key_state, *((self.vdata, self.vscales, self.vzeros) if C else (None,) * 3), self.rk, self.rv,
+            self.seq_lengths, self._next_lengths, qn.signs, qn.thresholds, *((qn.centroids, qn.gaussian, qn.gaussian_t)
+            if ip else (None,) * 3), ip, row0, C, self.bits, self.value_group_size, leaving, fill, _lib.stream_of(keys))
+        if past is None:
+            raise RuntimeError("TurboQuant append: keys/values must be plain device tensors of the cache's dtype")
         self.seq_lengths, self._next_lengths = self._next_lengths, self.seq_lengths
         return past
 
@@ -243,10 +223,27 @@ class _LayerSlab:
             self._ws[name] = t
         return t[:numel].view(shape)
 
+    def _decode_host(self, query, scaling, gate, rows):
+        qn = get_turboquant_quantizer(head_dim=self.head_dim, bits=self.bits, device=self.device)
+        ip, C = self.key_quantizer == "ip", self.capacity
+        fields = (None,) * 5 if C == 0 else (self.kdense if ip else self.kcodes, None if ip else self.knorms,
+                                             self.vdata, self.vscales, self.vzeros)
+        if rows != slice(None):
+            fields = tuple(None if t is None else t[rows] for t in fields)
+        rk, rv, lens = (self.rk, self.rv, self.seq_lengths) if rows == slice(None) else (
+            self.rk[rows], self.rv[rows], self.seq_lengths[rows])
+        return _lib.host().decode_rows(query, gate, None, *fields, rk, rv, lens, qn.rotation, qn.rotation_t, qn.centroids,
+                                       qn.signs, None, None, None, self.bits, self.value_group_size, scaling,
+                                       _DECODE_BLOCK_SIZE, not ip, _lib.stream_of(query))
+
     def decode(self, query: torch.Tensor, *, scaling: float, gate: torch.Tensor | None,
                rows: slice = slice(None)) -> torch.Tensor:
         """query [b, Hq, 1, D] for the sequences `rows` -> output of the same shape: one split-KV
         decode over [quantized slots ++ window ring] with the device lengths."""
+        if query.is_cuda and 0 not in self.lengths:
+            got = self._decode_host(query, scaling, gate, rows)
+            if got is not None:
+                return got
         b = query.shape[0]
         hq, D = int(query.shape[1]), self.head_dim
         C = self.capacity
