@@ -253,7 +253,8 @@ def load() -> ctypes.CDLL:
 
 _HOST_ENTRIES = ("anna_mi_last_error", "anna_mi_int4_linear", "anna_mi_decode_num_blocks", "anna_mi_gqa_decode_splitkv",
                  "anna_mi_tq_decode", "anna_mi_tq_store", "anna_mi_moe_route_small", "anna_mi_moe_gather",
-                 "anna_mi_moe_router", "anna_mi_moe_dispatch", "anna_mi_moe_grouped_int4_mlp", "anna_mi_moe_combine")
+                 "anna_mi_moe_router", "anna_mi_moe_dispatch", "anna_mi_moe_grouped_int4_mlp", "anna_mi_moe_combine",
+                 "anna_mi_moe_prefill_workspace", "anna_mi_moe_prefill")
 _host = None
 
 

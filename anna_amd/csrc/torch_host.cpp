@@ -42,6 +42,8 @@ struct Library {
   decltype(&anna_mi_moe_dispatch) moe_dispatch = nullptr;
   decltype(&anna_mi_moe_grouped_int4_mlp) moe_grouped_int4_mlp = nullptr;
   decltype(&anna_mi_moe_combine) moe_combine = nullptr;
+  decltype(&anna_mi_moe_prefill_workspace) moe_prefill_workspace = nullptr;
+  decltype(&anna_mi_moe_prefill) moe_prefill = nullptr;
 } lib;
 
 void bind(const py::dict& d) {
@@ -60,6 +62,8 @@ void bind(const py::dict& d) {
   get("anna_mi_moe_dispatch", lib.moe_dispatch);
   get("anna_mi_moe_grouped_int4_mlp", lib.moe_grouped_int4_mlp);
   get("anna_mi_moe_combine", lib.moe_combine);
+  get("anna_mi_moe_prefill_workspace", lib.moe_prefill_workspace);
+  get("anna_mi_moe_prefill", lib.moe_prefill);
 }
 
 void check(int rc, const char* name) {
@@ -387,6 +391,26 @@ OptTensor moe_block(const Tensor& x, const Tensor& logits, const Tensor& gq, con
   if (!is(experts, dev, at::kLong) || !is(slots, dev, at::kLong) || experts.numel() != E || slots.numel() != E)
     return std::nullopt;
   const int64_t I = gq.size(1);
+  if (x.stride(0) % 8 == 0 && (uintptr_t)ptr(x) % 16 == 0 && dq.size(1) == H && ds.size(2) == H && gs.size(2) == I) {
+    anna_mi_moe_prefill_args p{};
+    p.dtype = dt, p.logits_dtype = ldt, p.scale_dtype = sdt, p.normalize = normalize;
+    p.tokens = T, p.num_experts = E, p.top_k = top_k, p.hidden_dim = H, p.intermediate_dim = I, p.group_size = group;
+    p.hidden = ptr(x), p.hidden_row_stride = T > 1 ? x.stride(0) : std::max(H, x.stride(0));
+    p.logits = ptr(logits), p.logits_row_stride = logits.stride(0);
+    p.slots = (const int64_t*)ptr(slots);
+    p.gate_qweight = (const int32_t*)ptr(gq), p.gate_qscale = ptr(gs), p.gate_qzeros = (const int8_t*)ptr(gz);
+    p.up_qweight = (const int32_t*)ptr(uq), p.up_qscale = ptr(us), p.up_qzeros = (const int8_t*)ptr(uz);
+    p.down_qweight = (const int32_t*)ptr(dq), p.down_qscale = ptr(ds), p.down_qzeros = (const int8_t*)ptr(dz);
+    p.hidden_packed_cols = gq.size(2), p.hidden_groups = gs.size(1);
+    p.intermediate_packed_cols = dq.size(2), p.intermediate_groups = ds.size(1);
+    if (const int64_t bytes = lib.moe_prefill_workspace(&p); bytes > 0) {
+      Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte).requires_grad(false));
+      Tensor out = at::empty({T, H}, x.options().requires_grad(false));
+      p.workspace = ptr(ws), p.out = ptr(out);
+      check(lib.moe_prefill(&p, stream_ptr(stream)), "anna_mi_moe_prefill");
+      return out;
+    }
+  }
   const size_t es = (size_t)x.element_size();
   Carve c;
   const size_t o_w = c.take(R * 4), o_sel = c.take(R * 8), o_usage = c.take(E * 4), o_off = c.take((E + 1) * 8),

@@ -639,6 +639,31 @@ typedef struct {
 } anna_mi_moe_mlp_args;
 
 int64_t anna_mi_sizeof_moe_mlp_args(void);
+
+/* The whole routed block for many routes per expert (no single counterpart in the reference:
+ * _route_tokens, _sorted_routing_assignments, the grouped MLP and index_add_, ops.py:3280-3457), for
+ * 16-bit hidden states, group 128 and dims that are multiples of 128.  Every expert of the bank is
+ * active, slots[e] its slot. */
+typedef struct {
+  int dtype, logits_dtype, scale_dtype;
+  int normalize;
+  int64_t tokens, num_experts, top_k, hidden_dim, intermediate_dim, group_size;
+  const void* hidden;  /* [tokens][hidden_dim], row stride below */
+  int64_t hidden_row_stride;
+  const void* logits;  /* [tokens][num_experts] */
+  int64_t logits_row_stride;
+  const int64_t* slots;
+  const int32_t* gate_qweight; const void* gate_qscale; const int8_t* gate_qzeros; /* as anna_mi_moe_mlp_args */
+  const int32_t* up_qweight; const void* up_qscale; const int8_t* up_qzeros;
+  const int32_t* down_qweight; const void* down_qscale; const int8_t* down_qzeros;
+  int64_t hidden_packed_cols, hidden_groups, intermediate_packed_cols, intermediate_groups;
+  void* workspace;     /* anna_mi_moe_prefill_workspace bytes, 256-byte aligned */
+  void* out;           /* [tokens][hidden_dim] */
+} anna_mi_moe_prefill_args;
+/* Bytes of workspace, or 0: not a call of this form (shape, or too few routes per expert). */
+int64_t anna_mi_moe_prefill_workspace(const anna_mi_moe_prefill_args* args);
+int anna_mi_moe_prefill(const anna_mi_moe_prefill_args* args, void* stream);
+int64_t anna_mi_sizeof_moe_prefill_args(void);
 int anna_mi_moe_grouped_int4_mlp(const anna_mi_moe_mlp_args* args, void* stream);
 
 #ifdef __cplusplus

@@ -1,0 +1,81 @@
+"""The sparse block for many routes per expert (anna_mi_moe_prefill) against the fp64 brute force over the
+dequantized bank, and against the separate ops' routing."""
+
+import pytest
+import torch
+
+from anna_amd import _lib
+from anna_amd.moe import SparseMoeInt4
+from oracle import cpu_paths as cp
+from tests._util import BF16_TOL, rel_err
+from tests.test_moe_gpu import dequant_experts, make_bank
+
+pytestmark = pytest.mark.gpu
+
+
+def brute_force(bank, x, logits, top_k, norm):
+    w, sel, _ = cp.moe_route(logits.cpu(), top_k, norm)
+    out = torch.zeros(x.shape, dtype=torch.float64)
+    experts = dequant_experts(bank, sorted(set(sel.reshape(-1).tolist())))
+    xd = x.cpu().double()
+    for e, (wg, wu, wd) in experts.items():
+        t, k = (sel == e).nonzero(as_tuple=True)
+        g, u = xd[t] @ wg.double().t(), xd[t] @ wu.double().t()
+        out.index_add_(0, t, (torch.nn.functional.silu(g) * u) @ wd.double().t() * w[t, k].double().unsqueeze(1))
+    return out.numpy()
+
+
+# tokens x top_k / experts from 12 up: sweeps of one to three chunks, several sweeps, a ragged last tile
+# (intermediate 384 = 3 x 128, hidden 384 = 1.5 x 256), one group of K, the most groups of K, one
+# token per wave and several, tokens past one workgroup's share
+@pytest.mark.parametrize("tokens,experts,top_k,hidden,inter,dtype,scales,norm", [
+    (48, 4, 1, 128, 128, torch.bfloat16, torch.float32, True),
+    (61, 8, 2, 256, 384, torch.float16, torch.float32, True),
+    (200, 16, 4, 384, 256, torch.bfloat16, torch.bfloat16, False),
+    (333, 32, 8, 1024, 128, torch.bfloat16, torch.float16, True),
+    (130, 8, 8, 512, 640, torch.float16, torch.bfloat16, True),
+    (100, 8, 2, 4096, 128, torch.bfloat16, torch.float32, True),
+    (5003, 3, 1, 128, 128, torch.bfloat16, torch.float32, True),
+    (40, 64, 64, 256, 128, torch.bfloat16, torch.float32, False),
+])
+def test_prefill_block_matches_brute_force(gpu, tokens, experts, top_k, hidden, inter, dtype, scales, norm):
+    bank = make_bank(experts, hidden, inter, 128, scales, gpu, tokens)
+    torch.manual_seed(tokens)
+    wide = torch.randn(tokens, hidden + 64, device=gpu).to(dtype)
+    x = wide[:, :hidden]  # rows a stride apart
+    logits = torch.randn(tokens, experts, device=gpu)
+    block = SparseMoeInt4(bank, num_experts=experts, top_k=top_k, norm_topk_prob=norm)
+    ref = brute_force(bank, x, logits, top_k, norm)
+    assert rel_err(block(x, logits).double().cpu().numpy(), ref) <= BF16_TOL
+    # the reference's own 16-bit logits
+    block(x, logits.to(dtype))
+
+
+def test_prefill_block_skewed_experts(gpu):
+    """Experts without routes, one with a single route and one with nearly all of them (more sweeps than
+    workgroups were launched for)."""
+    experts, hidden, inter, tokens = 16, 256, 256, 700
+    bank = make_bank(experts, hidden, inter, 128, torch.float32, gpu, 1)
+    torch.manual_seed(5)
+    x = torch.randn(tokens, hidden, device=gpu, dtype=torch.bfloat16)
+    logits = torch.full((tokens, experts), -30.0, device=gpu)
+    logits[:, 3] = 5.0
+    logits[:, 9] = 4.0 + torch.rand(tokens, device=gpu) * 0.5
+    logits[17, 12] = 9.0
+    block = SparseMoeInt4(bank, num_experts=experts, top_k=2)
+    got = block(x, logits)
+    assert rel_err(got.double().cpu().numpy(), brute_force(bank, x, logits, 2, True)) <= BF16_TOL
+    assert torch.equal(got, block(x, logits))  # no atomics: the same bits again
+
+
+def test_prefill_takes_only_its_shapes(gpu):
+    """Group 64, fp32 hidden states, dims off 128 and few routes go the general way."""
+    torch.manual_seed(2)
+    for experts, hidden, inter, group, dtype, tokens in ((8, 256, 256, 64, torch.bfloat16, 64),
+                                                         (8, 256, 256, 128, torch.float32, 64),
+                                                         (32, 256, 256, 128, torch.bfloat16, 20)):
+        bank = make_bank(experts, hidden, inter, group, torch.float32, gpu, 3)
+        x = torch.randn(tokens, hidden, device=gpu).to(dtype)
+        logits = torch.randn(tokens, experts, device=gpu)
+        block = SparseMoeInt4(bank, num_experts=experts, top_k=2)
+        assert rel_err(block(x, logits).double().cpu().numpy(), brute_force(bank, x, logits, 2, True)) <= BF16_TOL
