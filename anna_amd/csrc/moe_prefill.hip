@@ -11,16 +11,21 @@
 //   moe_pf_gemm     the two products, below.
 //   moe_pf_combine  out[t] = sum of its routes' rows.
 //
-// moe_pf_gemm.  A 4-wave workgroup takes (expert, tile, sweep): 256 rows of W -- 128 of the gate and
-// the same of the up matrix, or 256 of the down matrix -- against up to 48 of the expert's routes (an
-// expert's 16-route chunks split evenly over its sweeps).  Each wave holds 64 rows of W as four MFMA
-// operands in registers, so that one read of an x operand from LDS feeds four instructions and a nibble
-// conversion up to three; two workgroups share a compute unit and fill each other's barriers and
-// waits.  K runs in passes of one group: W comes two passes ahead into a ring of the
-// wave's own in LDS, scales and zero points two passes ahead into registers, x one pass ahead through registers into a double-buffered, chunk-swizzled LDS tile, the sums of all
-// groups into LDS at the start.  The
-// scale and zero point are applied per group in fp32 as s (sum x (off + q) - (off + z) sum x); the
-// activation between the products is bf16, as in the other forms (moe.hip).
+// moe_pf_gemm.  A 4-wave workgroup takes (expert, item, sweep): an item is one or more consecutive tiles of
+// 256 rows of W -- 128 of the gate and the same of the up matrix, or 256 of the down matrix -- and a sweep
+// up to 48 of the expert's routes (its 16-route chunks split evenly over its sweeps).  Each wave holds 64
+// rows of W as four MFMA operands, so that one read of an x operand from LDS feeds four instructions and a
+// nibble conversion up to three; two workgroups share a compute unit and fill each other's barriers and
+// waits.  The steps of an item's tiles (one group of K each) form one pipeline: W two steps ahead into a
+// ring of the wave's own in LDS, x two steps ahead through registers into a double-buffered,
+// chunk-swizzled LDS tile, scales and zero points a step ahead in registers, the sums of all groups in
+// LDS from the start.  The scale and zero point are applied per group in fp32 as
+// s (sum x (off + q) - (off + z) sum x); the activation between the products is bf16, as in the other
+// forms (moe.hip).  What bounds it: issue, ~6.5 VALU instructions (conversion, scaling, addresses) to an
+// MFMA.  2048 tokens, 128 experts, top 8, 2048 x 512: gate/up 203 -> 161 us, down 109 -> 107, the block
+// 445 -> 320; 32 experts of 768 1060 -> 345.  Measured and not kept: 8 waves of two operands against
+// up to 128 routes in one workgroup per compute unit (181 + 140 us; W is converted once, but nothing fills
+// the barriers).
 #include <algorithm>
 #include <type_traits>
 
@@ -79,21 +84,29 @@ __global__ __launch_bounds__(64 * PF_RT_WAVES) void moe_pf_gather(
     const int32_t* __restrict__ selected, const int32_t* __restrict__ counts, const int64_t* __restrict__ slots,
     uint16_t* __restrict__ xg, float* __restrict__ sums, uint16_t* __restrict__ cw, int32_t* __restrict__ route_pos,
     int32_t* __restrict__ items) {
-  __shared__ int s_scan[16], s_first[512], s_sel[PF_RT_ROUTES], s_pos[PF_RT_ROUTES];
+  __shared__ int s_scan[16], s_first[512], s_before[512], s_sel[PF_RT_ROUTES], s_pos[PF_RT_ROUTES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int E = (int)p.experts, e = threadIdx.x, k = (int)p.top_k;
   const int64_t t0 = blockIdx.x * p.wg_tokens, t1 = t0 + p.wg_tokens < p.tokens ? t0 + p.wg_tokens : p.tokens;
   const int n = (int)(t1 - t0) * k;
   if (e < n) s_sel[e] = selected[t0 * k + e];
-  int total = 0, before = 0;
-  if (e < E) {
-#pragma unroll 8
-    for (int w = 0; w < (int)p.wgs; ++w) {
-      const int c = counts[(int64_t)w * E + e];
+  // expert counts of all ranges and of those before this one: 1024 / EP threads share an expert
+  const int EP = E <= 64 ? 64 : E <= 128 ? 128 : E <= 256 ? 256 : 512;
+  if (e < 512) s_first[e] = s_before[e] = 0;
+  __syncthreads();
+  if ((e & (EP - 1)) < E) {
+    int total = 0, before = 0;
+#pragma unroll 16
+    for (int w = e / EP; w < (int)p.wgs; w += 1024 / EP) {
+      const int c = counts[(int64_t)w * E + (e & (EP - 1))];
       total += c;
       before += w < (int)blockIdx.x ? c : 0;
     }
+    atomicAdd(&s_first[e & (EP - 1)], total);
+    atomicAdd(&s_before[e & (EP - 1)], before);
   }
+  __syncthreads();
+  const int total = e < E ? s_first[e] : 0, before = e < E ? s_before[e] : 0;
   int all, nact;
   const int start = block_exclusive_scan(total, s_scan, &all);
   const int j = block_exclusive_scan(total > 0 ? 1 : 0, s_scan, &nact);
@@ -151,7 +164,8 @@ struct PfGemm {
   const int8_t* qz[2];
   int64_t N, K, pc, routes;  // rows and columns of a matrix, packed words per row
   uint32_t slot_bytes_w;     // bytes of a slot's matrix
-  int sweeps;                // workgroups per (expert, tile)
+  int sweeps;                // workgroups per (expert, item)
+  int tiles;                 // consecutive tiles of an item: one pipeline over their steps
   uint16_t* out;             // act [routes][N] bf16 interleaved, or [routes][N] in the hidden dtype
   float* act_sums;           // gate/up: [N / 128][routes]
 };
@@ -164,7 +178,7 @@ struct PfScales {
 
 template <int HDT, int SDT, bool GU, int NC>
 __device__ __forceinline__ void pf_sweep(const PfGemm& a, uint16_t* xs, unsigned char* ws, float* s_x, float (*s_sum)[16 * PF_NC],
-                                         uint32_t slot, int tile, int64_t c0, int R) {
+                                         uint32_t slot, int tile0, int ntile, int64_t c0, int R) {
   constexpr int MDT = GU ? HDT : ANNA_MI_BF16;
   constexpr float OFF = MDT == ANNA_MI_BF16 ? 128.0f : 1024.0f;
   using ST = typename Elem<SDT>::T;
@@ -175,7 +189,7 @@ __device__ __forceinline__ void pf_sweep(const PfGemm& a, uint16_t* xs, unsigned
   int nf[4];
 #pragma unroll
   for (int f = 0; f < 4; ++f)
-    nf[f] = GU ? tile * 128 + wave * 32 + 16 * (f & 1) + r : tile * 256 + wave * 64 + 16 * f + r;
+    nf[f] = GU ? tile0 * 128 + wave * 32 + 16 * (f & 1) + r : tile0 * 256 + wave * 64 + 16 * f + r;
   __amdgpu_buffer_rsrc_t rw[2], rs[2], rz[2];
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
@@ -186,13 +200,12 @@ __device__ __forceinline__ void pf_sweep(const PfGemm& a, uint16_t* xs, unsigned
                                               (int)(G * N * sizeof(ST)), 0x00020000);
     rz[m] = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(a.qz[q]) + (uint64_t)slot * G * N, 0, G * N, 0x00020000);
   }
-  // rows past N read as zero (offset past the buffer) and are not stored
-  uint32_t wo[4], so[4];
+  // rows past N read other rows' scales and no weights (past the buffer: zero), and are not stored
+  constexpr int ROWS = GU ? PF_ROWS / 2 : PF_ROWS;
+  const int tile_w = ROWS * (int)a.pc * 4;
+  uint32_t wo[4];
 #pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    wo[f] = nf[f] < N ? (uint32_t)((nf[f] * (int)a.pc + kq * 4) * 4) : 0x80000000u;
-    so[f] = nf[f] < N ? (uint32_t)nf[f] : 0x40000000u;
-  }
+  for (int f = 0; f < 4; ++f) wo[f] = (uint32_t)((nf[f] * (int)a.pc + kq * 4) * 4);
   // x: chunk i of this thread is row (t + 256 i) / 16, 16-byte chunk (t + 256 i) % 16 of the pass; rows
   // past the sweep's repeat the last one (their results are not stored)
   // (32-bit offsets from the sweep's first row)
@@ -208,36 +221,48 @@ __device__ __forceinline__ void pf_sweep(const PfGemm& a, uint16_t* xs, unsigned
   }
   // W of group g into stage st of the wave's ring (every lane reads back its own 16 bytes)
   unsigned char* const wl = ws + wave * (3 * 4096);
-  auto load = [&](int g, int st, PfScales<SDT>& P) {
-    g = g < G ? g : G - 1;
+  // a step: group g of tile t (past the last one: the last one again)
+  struct Step {
+    int t, g;
+  };
+  auto advance = [&](Step& p) {
+    if (p.g + 1 < G) ++p.g;
+    else if (p.t + 1 < ntile) ++p.t, p.g = 0;
+  };
+  auto load = [&](const Step& p, int st, u32x4 (&xr)[NC]) {
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       const int m = GU ? f >> 1 : 0;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw[m], (pf_lds_ptr)(wl + st * 4096 + f * 1024), 16, wo[f], g * 64, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw[m], (pf_lds_ptr)(wl + st * 4096 + f * 1024), 16, wo[f],
+                                               p.t * tile_w + p.g * 64, 0, 0);
     }
+    __builtin_amdgcn_sched_barrier(0);  // W of a step is requested before its x (see pass)
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      xr[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xo[i], p.g * 256, 0));
+  };
+  auto load_scales = [&](const Step& p, PfScales<SDT>& P) {
+    const int row = p.g * N + p.t * ROWS;
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       const int m = GU ? f >> 1 : 0;
-      if constexpr (sizeof(ST) == 4) P.s[f] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs[m], so[f] * 4, g * N * 4, 0));
-      else P.s[f] = (ST)__builtin_amdgcn_raw_buffer_load_b16(rs[m], so[f] * 2, g * N * 2, 0);
-      P.z[f] = (int8_t)__builtin_amdgcn_raw_buffer_load_b8(rz[m], so[f], g * N, 0);
+      if constexpr (sizeof(ST) == 4) P.s[f] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs[m], nf[f] * 4, row * 4, 0));
+      else P.s[f] = (ST)__builtin_amdgcn_raw_buffer_load_b16(rs[m], nf[f] * 2, row * 2, 0);
+      P.z[f] = (int8_t)__builtin_amdgcn_raw_buffer_load_b8(rz[m], nf[f], row, 0);
     }
   };
-  u32x4 xr[NC];
-  auto load_x = [&](int g) {
-    g = g < G ? g : G - 1;
-#pragma unroll
-    for (int i = 0; i < NC; ++i) xr[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xo[i], g * 256, 0));
-  };
-  auto store_x = [&](int buf) {
+  auto store_x = [&](const u32x4 (&xr)[NC], int buf) {
 #pragma unroll
     for (int i = 0; i < NC; ++i) *(u32x4*)(xs + buf * (16 * PF_NC * 128) + xl[i]) = xr[i];
   };
   f32x4 out[NC][4];
+  auto clear = [&]() {
 #pragma unroll
-  for (int c = 0; c < NC; ++c)
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int f = 0; f < 4; ++f) out[c][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int f = 0; f < 4; ++f) out[c][f] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
   auto compute = [&](const PfScales<SDT>& P, int g, int st, int buf) {
     u32x4 wq[4];
 #pragma unroll
@@ -248,22 +273,17 @@ __device__ __forceinline__ void pf_sweep(const PfGemm& a, uint16_t* xs, unsigned
     for (int c = 0; c < NC; ++c)
 #pragma unroll
       for (int f = 0; f < 4; ++f) acc[c][f] = f32x4{0.f, 0.f, 0.f, 0.f};
-    u32x4 xa[2][NC];
-    auto read = [&](int s) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c) xa[s & 1][c] = *(const u32x4*)(xb + c * 16 * 128 + (((kq * 4 + s) ^ r) * 8));
-    };
-    read(0);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      if (s < 3) read(s + 1);
-      u32x4 wf[4];
+      u32x4 wf[4], xa[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) xa[c] = *(const u32x4*)(xb + c * 16 * 128 + (((kq * 4 + s) ^ r) * 8));
 #pragma unroll
       for (int f = 0; f < 4; ++f) wf[f] = nibbles_to_frag<MDT>(wq[f][s]);
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
-        for (int f = 0; f < 4; ++f) acc[c][f] = mfma16<MDT>(xa[s & 1][c], wf[f], acc[c][f]);
+        for (int f = 0; f < 4; ++f) acc[c][f] = mfma16<MDT>(xa[c], wf[f], acc[c][f]);
     }
     f32x4 sx[NC];
 #pragma unroll
@@ -279,76 +299,101 @@ __device__ __forceinline__ void pf_sweep(const PfGemm& a, uint16_t* xs, unsigned
   };
   // LDS writes done, then the barrier (the loads ahead stay in flight)
   auto meet = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  PfScales<SDT> A, B, C;
-  load(0, 0, A);
-  load_x(0);
-  load(1, 1, B);
+  // C layout: lane (r, kq) element i is route c0 + 16 c + 4 kq + i of W row nf (of tile t)
+  auto finish = [&](int t) {
+    int base = (int)c0, left = R, nn = N;
+    asm volatile("" : "+s"(base), "+s"(left), "+s"(nn));
+    if constexpr (GU) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = 16 * c + 4 * kq + i;
+          float both = 0.f;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int n = nf[h] + t * ROWS;
+            const uint16_t v = f32_to_bf16_bits(pf_silu(out[c][h][i]) * out[c][h + 2][i]);
+            both += n < nn ? bf16_bits_to_f32(v) : 0.f;
+            if (m < left && n < nn) a.out[(int64_t)(base + m) * nn + (n & ~7) + pf_pos(n & 7)] = v;
+          }
+          both += dpp_move<0xB1>(both);
+          both += dpp_move<0x4E>(both);
+          both += dpp_move<0x141>(both);
+          both += dpp_move<0x140>(both);
+          if (r == 0) s_sum[wave][m] = both;
+        }
+      __syncthreads();
+      if ((int)threadIdx.x < left)
+        a.act_sums[(int64_t)(tile0 + t) * a.routes + c0 + threadIdx.x] =
+            (s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x]) + (s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x]);
+    } else {
+      using HT = typename Elem<HDT>::T;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = 16 * c + 4 * kq + i;
+          if (m >= left) continue;
+          const float wr = s_sum[0][m];  // the routing weight
+#pragma unroll
+          for (int f = 0; f < 4; ++f) {
+            const int n = nf[f] + t * ROWS;
+            if (n < nn) ((HT*)a.out)[(int64_t)(base + m) * nn + n] = Elem<HDT>::cvt(out[c][f][i] * wr);
+          }
+        }
+    }
+  };
+  PfScales<SDT> A, B;
+  u32x4 XA[NC], XB[NC];
+  Step ahead1{0, 0}, ahead2{0, 0};  // the steps whose scales, and whose W and x, are requested next
+  load_scales(ahead1, A);
+  advance(ahead1);
+  load(ahead2, 0, XA);
+  advance(ahead2);
+  __builtin_amdgcn_sched_barrier(0);
+  load(ahead2, 1, XB);
+  advance(ahead2);
+  __builtin_amdgcn_sched_barrier(0);
   for (int i = threadIdx.x; i < G * 16 * NC; i += 64 * PF_WAVES) {
     const int g = i / (16 * NC), m = i - g * (16 * NC);
     s_x[g * (16 * PF_NC) + m] = m < R ? a.sums[(int64_t)g * a.routes + c0 + m] : 0.f;
   }
-  store_x(0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // W of group 0 (here nothing orders it before x)
+  if constexpr (!GU) {
+    if ((int)threadIdx.x < R) s_sum[0][threadIdx.x] = Elem<HDT>::to_f32(a.cw[c0 + threadIdx.x]);
+  }
+  store_x(XA, 0);
   meet();
-  // pass g: request x of g + 1, then W of g + 2 (into the stage pass g - 1 read), compute g, publish x of
-  // g + 1 (its buffer was last read in pass g - 1).  Loads complete in order, so a wave that has x of
-  // group g in registers has W of group g in its ring: x of g is requested after it and waited for
-  // before the barrier that ends pass g - 1.
-  auto pass = [&](int g, int st, const PfScales<SDT>& cur, PfScales<SDT>& ahead) {
-    load_x(g + 1);
-    load(g + 2, st == 0 ? 2 : st - 1, ahead);
+  // Step q (group g of tile t): request the scales of q + 1, then W and x of q + 2 (W into the stage step
+  // q - 1 read), compute q, publish x of q + 1 (its buffer was last read in step q - 1).  Loads complete in
+  // order and a step's W is requested before its x, so a wave that has x of a step in registers, as it must
+  // to publish it a step ahead, has the step's W in its ring.
+  const int steps = ntile * G;
+  int t = 0, g = 0, st = 0;
+  auto pass = [&](int buf, const PfScales<SDT>& cur, PfScales<SDT>& next, const u32x4 (&xnext)[NC], u32x4 (&xahead)[NC]) {
+    load_scales(ahead1, next);
+    advance(ahead1);
+    load(ahead2, st == 0 ? 2 : st - 1, xahead);
+    advance(ahead2);
     __builtin_amdgcn_sched_barrier(0);
-    compute(cur, g, st, g & 1);
-    store_x((g + 1) & 1);
+    compute(cur, g, st, buf);
+    st = st == 2 ? 0 : st + 1;
+    if (++g == G) {
+      finish(t);
+      clear();
+      g = 0, ++t;
+    }
+    store_x(xnext, buf ^ 1);
     meet();
   };
-  for (int g = 0; g < G; g += 3) {
-    pass(g, 0, A, C);
-    if (g + 1 < G) pass(g + 1, 1, B, A);
-    if (g + 2 < G) pass(g + 2, 2, C, B);
+  for (int q = 0; q < steps; q += 2) {
+    pass(0, A, B, XB, XA);
+    if (q + 1 < steps) pass(1, B, A, XA, XB);
   }
-  // the last passes' clamped copies land in stages nobody reads; before the next sweep's first ones
+  // the last steps' repeated copies land in stages nobody reads: before the next sweep's first ones; and
+  // s_sum is free
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  // C layout: lane (r, kq) element i is route c0 + 16 c + 4 kq + i of W row nf
-  if constexpr (GU) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = 16 * c + 4 * kq + i;
-        float both = 0.f;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const uint16_t v = f32_to_bf16_bits(pf_silu(out[c][h][i]) * out[c][h + 2][i]);
-          both += nf[h] < N ? bf16_bits_to_f32(v) : 0.f;
-          if (m < R && nf[h] < N) a.out[(c0 + m) * N + (nf[h] & ~7) + pf_pos(nf[h] & 7)] = v;
-        }
-        both += dpp_move<0xB1>(both);
-        both += dpp_move<0x4E>(both);
-        both += dpp_move<0x141>(both);
-        both += dpp_move<0x140>(both);
-        if (r == 0) s_sum[wave][m] = both;
-      }
-    __syncthreads();
-    if ((int)threadIdx.x < R)
-      a.act_sums[(int64_t)tile * a.routes + c0 + threadIdx.x] =
-          (s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x]) + (s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x]);
-    __syncthreads();  // s_sum and the x buffers are free for the next sweep
-  } else {
-    using HT = typename Elem<HDT>::T;
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = 16 * c + 4 * kq + i;
-        if (m >= R) continue;
-        const float wr = Elem<HDT>::to_f32(a.cw[c0 + m]);
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-          if (nf[f] < N) ((HT*)a.out)[(c0 + m) * N + nf[f]] = Elem<HDT>::cvt(out[c][f][i] * wr);
-      }
-    __syncthreads();
-  }
+  __syncthreads();
 }
 
 template <int HDT, int SDT, bool GU>
@@ -359,7 +404,8 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void moe_pf_gemm(const PfGemm a) 
   float(*const s_sum)[16 * PF_NC] = (float(*)[16 * PF_NC])(ws + PF_W_BYTES);
   float* const s_x = (float*)(ws + PF_W_BYTES + PF_S_BYTES);
   const int nact = a.items[0];
-  const int rows = GU ? PF_ROWS / 2 : PF_ROWS, tiles = ((int)a.N + rows - 1) / rows;
+  const int rows = GU ? PF_ROWS / 2 : PF_ROWS, all = ((int)a.N + rows - 1) / rows;
+  const int tiles = (all + a.tiles - 1) / a.tiles;  // items of a.tiles consecutive tiles
   // expert-major within a (tile, sweep): an expert's workgroups are nact apart, on one XCD where nact
   // is a multiple of 8, and share its L2 copy of the expert's x and W
   const int total = nact * tiles * a.sweeps;
@@ -372,10 +418,11 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void moe_pf_gemm(const PfGemm a) 
     for (int sw = rest / tiles; sw < nsw; sw += a.sweeps) {
       const int lo = sw * chunks / nsw, hi = (sw + 1) * chunks / nsw;
       const int64_t c0 = start + 16 * lo;
+      const int t0 = tile * a.tiles, nt = all - t0 < a.tiles ? all - t0 : a.tiles;
       const int R = (start + 16 * hi < end ? start + 16 * hi : end) - (int)c0;
-      if (hi - lo == 1) pf_sweep<HDT, SDT, GU, 1>(a, xs, ws, s_x, s_sum, slot, tile, c0, R);
-      else if (hi - lo == 2) pf_sweep<HDT, SDT, GU, 2>(a, xs, ws, s_x, s_sum, slot, tile, c0, R);
-      else pf_sweep<HDT, SDT, GU, 3>(a, xs, ws, s_x, s_sum, slot, tile, c0, R);
+      if (hi - lo == 1) pf_sweep<HDT, SDT, GU, 1>(a, xs, ws, s_x, s_sum, slot, t0, nt, c0, R);
+      else if (hi - lo == 2) pf_sweep<HDT, SDT, GU, 2>(a, xs, ws, s_x, s_sum, slot, t0, nt, c0, R);
+      else pf_sweep<HDT, SDT, GU, 3>(a, xs, ws, s_x, s_sum, slot, t0, nt, c0, R);
     }
   }
 }
@@ -468,12 +515,12 @@ using namespace anna;
 
 extern "C" int64_t anna_mi_sizeof_moe_prefill_args(void) { return (int64_t)sizeof(anna_mi_moe_prefill_args); }
 
-// From 12 routes per expert on average.  Below, a sweep's chunk is mostly padding and the forms of moe.hip
-// that keep all of K resident are as fast.
+// From 18 routes per expert on average: 300 tokens of 64 experts, top 4 (18.75) 51 against 54 us with the
+// forms of moe.hip, 64 tokens of 32 experts, top 8 (16) 50 against 46, 128 experts, top 8: 64 tokens (4) 96
+// against 88, 128 tokens (8) 100 against 101, 512 tokens (32) 137 against 161, 2048 (128) 320 against 440.
 extern "C" int64_t anna_mi_moe_prefill_workspace(const anna_mi_moe_prefill_args* ap) {
   if (!ap || !pf_shape_ok(*ap)) return 0;
-  static const int64_t min_routes = getenv("LAB_PF_MIN") ? atoi(getenv("LAB_PF_MIN")) : 12;
-  if (ap->tokens * ap->top_k < min_routes * ap->num_experts) return 0;
+  if (ap->tokens * ap->top_k < 18 * ap->num_experts) return 0;
   return pf_layout(pf_plan(*ap)).total;
 }
 
@@ -519,7 +566,10 @@ extern "C" int anna_mi_moe_prefill(const anna_mi_moe_prefill_args* ap, void* str
     g.sweeps = (int)std::max<int64_t>(1, (p.routes * 3 / 2 / a.num_experts + 16 * PF_NC - 1) / (16 * PF_NC));
     auto launch = [&](auto gu_tag) {
       constexpr bool GU = decltype(gu_tag)::value;
-      const int64_t tiles = (g.N + (GU ? 127 : 255)) / (GU ? 128 : 256);
+      // an item's steps fill the pipeline once: eight of them or more (the down product at K = 512: 132 us
+      // with 4 steps, 113 with 8, 107 with 16, which loses where items are few: 372 against 345 us a block)
+      g.tiles = (int)std::max<int64_t>(1, (8 * 128 + g.K - 1) / g.K);
+      const int64_t all = (g.N + (GU ? 127 : 255)) / (GU ? 128 : 256), tiles = (all + g.tiles - 1) / g.tiles;
       const int64_t wgs = std::min<int64_t>(a.num_experts * tiles * g.sweeps, 1 << 16);
       auto kern = moe_pf_gemm<HDT, SDT, GU>;
       ANNA_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,

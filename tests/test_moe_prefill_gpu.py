@@ -25,12 +25,12 @@ def brute_force(bank, x, logits, top_k, norm):
     return out.numpy()
 
 
-# tokens x top_k / experts from 12 up: sweeps of one to three chunks, several sweeps, a ragged last tile
+# tokens x top_k / experts from 18 up: sweeps of one to three chunks, several sweeps, a ragged last tile
 # (intermediate 384 = 3 x 128, hidden 384 = 1.5 x 256), one group of K, the most groups of K, one
 # token per wave and several, tokens past one workgroup's share
 @pytest.mark.parametrize("tokens,experts,top_k,hidden,inter,dtype,scales,norm", [
-    (48, 4, 1, 128, 128, torch.bfloat16, torch.float32, True),
-    (61, 8, 2, 256, 384, torch.float16, torch.float32, True),
+    (73, 4, 1, 128, 128, torch.bfloat16, torch.float32, True),
+    (75, 8, 2, 256, 384, torch.float16, torch.float32, True),
     (200, 16, 4, 384, 256, torch.bfloat16, torch.bfloat16, False),
     (333, 32, 8, 1024, 128, torch.bfloat16, torch.float16, True),
     (130, 8, 8, 512, 640, torch.float16, torch.bfloat16, True),
