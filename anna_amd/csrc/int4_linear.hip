@@ -28,6 +28,7 @@
 //                    workgroup to bf16 ((q - z) * s rounded to bf16, the reference's
 //                    dequant numerics) next to a 128x128 tile of x, and 4 waves run
 //                    v_mfma_f32_32x32x16_bf16 on it.
+//   (groups of 32 or 64 that the GEMM does not take, and x that is not 16-byte aligned: int4_rows.hip)
 //   int4_linear_generic  any dtype / group / alignment; VALU, one wave per output row.
 #include <stdlib.h>
 
@@ -905,6 +906,9 @@ extern "C" int anna_mi_int4_linear(const void* x, int x_dtype, int64_t M, int64_
     ANNA_LAUNCH_CHECK("int4_gemm_mfma");
     return ANNA_MI_OK;
   }
+  // groups of 32 or 64, and x that is not 16-byte aligned (odd K or row stride)
+  if (int4_rows_supported(x_dtype, M, N, K, xs, qweight, pc, G, gsz))
+    return int4_rows_launch(x, x_dtype, M, K, xs, qweight, N, pc, qscale, scale_dtype, qzeros, G, gsz, y, st);
   dim3 grid((unsigned)N, (unsigned)((M + 7) / 8 < 64 ? (M + 7) / 8 : 64), 1);
   ANNA_DISPATCH_DTYPE(x_dtype, XDT, {
     ANNA_DISPATCH_DTYPE(scale_dtype, SDT, {
