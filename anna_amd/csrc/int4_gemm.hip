@@ -639,6 +639,12 @@ int int4_gemm_tiled_launch(const void* x, int x_dtype, int64_t M, int64_t K, int
   // likewise the middle tile at exactly one round (M = 256, N = 12288: 52.4 -> 46.4 us; M = 192:
   // 51.3 -> 43.9 us), whose one-step periods need an even step count
   const bool msplit = tiles(TileM{}) <= 256 && (K / GM_BK) % (2 * TileM2::SPB) == 0;
+  // Two small-tile workgroups share a compute unit, so that up to 512 of their tiles run in one round;
+  // past that, and below a round of middle tiles, the middle tile with K split is faster.  M = 333:
+  // K = 4096, N = 6144 (768 small tiles) 52.0 -> 38.3 us, K = 1024, N = 4096 (516) 16.9 -> 14.3; M = 1000,
+  // K = N = 2048 (688) 26.9 -> 22.2; with no more than 512 the small tile stays: M = 257, K = 1024,
+  // N = 4096 (430) 11.9 against 14.2 us, M = 700, K = N = 2048 (473) 18.3 against 21.2.
+  if (shape == 2 && msplit && tiles(TileS{}) > 512) shape = 1;
   // ANNA_MI_INT4_GEMM_TILE = L / M / S forces a tile shape (read on every call; the tests run
   // every shape on shapes small enough for the CPU oracle)
   if (const char* f = getenv("ANNA_MI_INT4_GEMM_TILE"); f && *f) shape = f[0] == 'L' ? 0 : f[0] == 'M' ? 1 : 2;

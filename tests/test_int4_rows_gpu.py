@@ -73,3 +73,20 @@ def test_rows_keep_infinities(gpu, m):
     want = w[:, 77] * float("inf")
     torch.testing.assert_close(out[0].cpu().double(), want, equal_nan=True)
     assert bool(torch.isfinite(out[1:]).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(193, 8832, 256), (385, 6000, 512)])
+def test_gemm_middle_tile_past_a_round_of_small_tiles(gpu, monkeypatch, m, n, k):
+    """More than 512 small tiles on less than a round of middle ones: the middle tile with K split."""
+    monkeypatch.delenv("ANNA_MI_INT4_GEMM_TILE", raising=False)
+    g = torch.Generator().manual_seed(m)
+    qw, qs, qz = _payload(g, n, k, 128, torch.float32)
+    qz.clamp_(0, 15)
+    x = torch.randn((m, k), generator=g).to(torch.bfloat16)
+    w = _weight(qw, qs, qz, k, 128)
+    ref = x.double() @ w.t()
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=gpu)
+    fused_ops.int4_linear_out(x.to(gpu), qw.to(gpu), qs.to(gpu), qz.to(gpu), 128, k, out)
+    # W rounded to bf16 and the result: 2^-9 each of their magnitudes
+    bound = ref.abs() * 2.0 ** -8 + (x.double().abs() @ w.abs().t()) * (2.0 ** -9 + (k + 8) * 2.0 ** -24)
+    assert bool(((out.cpu().double() - ref).abs() <= bound).all())
