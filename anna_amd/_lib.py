@@ -170,6 +170,21 @@ class MoeMlpArgs(ctypes.Structure):
     ]
 
 
+class MoePrefillArgs(ctypes.Structure):
+    """anna_mi_moe_prefill_args."""
+
+    _fields_ = [
+        ("dtype", _I), ("logits_dtype", _I), ("scale_dtype", _I), ("normalize", _I), ("tokens", _I64),
+        ("num_experts", _I64), ("top_k", _I64), ("hidden_dim", _I64), ("intermediate_dim", _I64), ("group_size", _I64),
+        ("hidden", _P), ("hidden_row_stride", _I64), ("logits", _P), ("logits_row_stride", _I64), ("slots", _P),
+        ("gate_qweight", _P), ("gate_qscale", _P), ("gate_qzeros", _P),
+        ("up_qweight", _P), ("up_qscale", _P), ("up_qzeros", _P),
+        ("down_qweight", _P), ("down_qscale", _P), ("down_qzeros", _P),
+        ("hidden_packed_cols", _I64), ("hidden_groups", _I64), ("intermediate_packed_cols", _I64),
+        ("intermediate_groups", _I64), ("workspace", _P), ("out", _P),
+    ]
+
+
 PROTOTYPES.update({
     "anna_mi_moe_router": [_P, _I, _I64, _I64, _I64, _I64, _I, _P, _P, _P, _P],
     "anna_mi_moe_dispatch": [_P, _I, _I64, _I64, _I64, _P, _I, _P, _P, _I, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P,
@@ -179,6 +194,7 @@ PROTOTYPES.update({
     "anna_mi_moe_scatter": [_P, _I, _I64, _I64, _P, _I64, _P, _P, _P],
     "anna_mi_moe_combine": [_P, _I, _I64, _P, _I64, _I64, _P, _P],
     "anna_mi_moe_grouped_int4_mlp": [ctypes.POINTER(MoeMlpArgs), _P],
+    "anna_mi_moe_prefill": [ctypes.POINTER(MoePrefillArgs), _P],
     "anna_mi_int4_gemv_tiled": [_P, _I, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _I, _P, _I64, _I64, _I64, _I64,
                                 _I64, _P, _I, _I64, _P],
     "anna_mi_topk_rows": [_P, _I64, _I64, _I64, _I64, _P, _I, _P, _P],
@@ -190,6 +206,8 @@ PROTOTYPES.update({
 # entry points that do not return a status code
 RAW_PROTOTYPES: dict[str, tuple] = {
     "anna_mi_sizeof_moe_mlp_args": (_I64, []),
+    "anna_mi_sizeof_moe_prefill_args": (_I64, []),
+    "anna_mi_moe_prefill_workspace": (_I64, [ctypes.POINTER(MoePrefillArgs)]),
     "anna_mi_decode_num_blocks": (_I64, [ctypes.POINTER(DecodeArgs)]),
     "anna_mi_sizeof_decode_args": (_I64, []),
     "anna_mi_gqa_decode_splitkv_noalloc_capacity": (_I64, []),
@@ -218,6 +236,8 @@ def _check_stamp(lib: ctypes.CDLL) -> None:
         raise RuntimeError(
             f"{LIB_PATH.name} is stale: built from sources {built[:12]}, the tree holds {want[:12]}; "
             "run `python -m anna_amd.build`")
+
+
 _lib: ctypes.CDLL | None = None
 
 

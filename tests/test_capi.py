@@ -43,6 +43,7 @@ def test_decode_args_binding_matches_the_c_struct():
     assert _lib.load().anna_mi_sizeof_tq_rows_append_args() == ctypes.sizeof(_lib.TQRowsAppendArgs)
     assert _lib.load().anna_mi_sizeof_tq_store_args() == ctypes.sizeof(_lib.TQStoreArgs)
     assert _lib.load().anna_mi_sizeof_tq_load_args() == ctypes.sizeof(_lib.TQLoadArgs)
+    assert _lib.load().anna_mi_sizeof_moe_prefill_args() == ctypes.sizeof(_lib.MoePrefillArgs)
 
 
 def test_library_is_stamped_with_the_tree_sources():
