@@ -14,6 +14,9 @@ __host__ __device__ constexpr int route_scratch(int64_t E) { return (int)((E + 3
 // cross-lane argmax: the probabilities go to the wave's LDS scratch sp (route_scratch(E)
 // floats), every lane counts for each of its experts how many experts beat it (a larger
 // probability, or an equal one at a lower index), and an expert of rank j < top_k is route j.
+// Every logit row gives top_k different experts: a row with a NaN or +inf logit, whose
+// probabilities are all NaN, ranks each of them as -1 (below every probability, ties by index) and
+// returns NaN weights, so that it spoils its own token only.
 // MAXV: experts per lane, E <= 64 MAXV (instantiated for E <= 64, 128, 256 and 1024).
 template <int LDT, int MAXV>
 __device__ __forceinline__ void route_token(const typename Elem<LDT>::T* __restrict__ logits, int64_t t, int64_t E,
@@ -42,7 +45,8 @@ __device__ __forceinline__ void route_token(const typename Elem<LDT>::T* __restr
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
     const int e = lane + 64 * i;
-    if (e < E) sp[e] = v[i] * inv;
+    const float p = v[i] * inv;
+    if (e < E) sp[e] = p == p ? p : -1.0f;
     else if (e < E4) sp[e] = -2.0f;     // padding: beats nothing, ties nothing
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -57,7 +61,7 @@ __device__ __forceinline__ void route_token(const typename Elem<LDT>::T* __restr
               (q.z > p || (q.z == p && j + 2 < e)) + (q.w > p || (q.w == p && j + 3 < e));
     }
     if (rank < top_k) {
-      stp[rank] = p;
+      stp[rank] = p < 0.f ? __builtin_nanf("") : p;
       ste[rank] = e;
     }
   }
