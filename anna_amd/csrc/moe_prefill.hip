@@ -416,7 +416,9 @@ __global__ __launch_bounds__(64 * PF_WAVES, 2) void moe_pf_gemm(const PfGemm a) 
     const int start = __builtin_amdgcn_readfirstlane(e.y), end = __builtin_amdgcn_readfirstlane(e.z);
     const int chunks = (end - start + 15) / 16, nsw = (chunks + PF_NC - 1) / PF_NC;
     for (int sw = rest / tiles; sw < nsw; sw += a.sweeps) {
-      const int lo = sw * chunks / nsw, hi = (sw + 1) * chunks / nsw;
+      // an even split whose terms stay below chunks (sw * chunks / nsw passes 2^31 from 1.3 M routes on)
+      const int each = chunks / nsw, more = chunks - each * nsw;
+      const int lo = sw * each + (sw < more ? sw : more), hi = lo + each + (sw < more ? 1 : 0);
       const int64_t c0 = start + 16 * lo;
       const int t0 = tile * a.tiles, nt = all - t0 < a.tiles ? all - t0 : a.tiles;
       const int R = (start + 16 * hi < end ? start + 16 * hi : end) - (int)c0;

@@ -79,3 +79,16 @@ def test_prefill_takes_only_its_shapes(gpu):
         logits = torch.randn(tokens, experts, device=gpu)
         block = SparseMoeInt4(bank, num_experts=experts, top_k=2)
         assert rel_err(block(x, logits).double().cpu().numpy(), brute_force(bank, x, logits, 2, True)) <= BF16_TOL
+
+
+def test_prefill_block_one_expert_past_a_million_routes(gpu):
+    """87,500 chunks in 29,167 sweeps of one expert: the same bits as in calls of 100,000 tokens."""
+    bank = make_bank(1, 128, 128, 128, torch.float32, gpu, 7)
+    tokens = 1_400_000
+    g = torch.Generator(device=gpu).manual_seed(9)
+    x = torch.randn(tokens, 128, device=gpu, generator=g).to(torch.bfloat16)
+    logits = torch.zeros(tokens, 1, device=gpu)
+    block = SparseMoeInt4(bank, num_experts=1, top_k=1)
+    got = block(x, logits)
+    for a in range(0, tokens, 100_000):
+        assert torch.equal(got[a:a + 100_000], block(x[a:a + 100_000], logits[a:a + 100_000]))
