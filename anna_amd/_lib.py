@@ -123,7 +123,7 @@ class TQStoreArgs(ctypes.Structure):
         ("value_data", _P), ("value_scales", _P), ("value_zeros", _P), ("residual_key", _P), ("residual_value", _P),
         ("seq_in", _P), ("seq_out", _P), ("past_out", _P), ("max_leaving", _I64), ("max_fill", _I64),
         ("signs", _P), ("thresholds", _P), ("centroids", _P), ("gaussian", _P), ("gaussian_t", _P),
-        ("value_lane_groups", _I), ("k0", _F),
+        ("value_lane_groups", _I), ("k0", _F), ("seq_lengths", _P),
     ]
 
 

@@ -302,7 +302,8 @@ OptTensor decode_pool(const Tensor& q, const OptTensor& gate, const OptTensor& o
 OptTensor tq_store(const Tensor& k, const Tensor& v, const OptTensor& key_codes, const OptTensor& key_norms,
                    const OptTensor& key_signs, const OptTensor& key_residual_norms, const OptTensor& key_dense,
                    const OptTensor& vdata, const OptTensor& vscales, const OptTensor& vzeros, const Tensor& rk,
-                   const Tensor& rv, const Tensor& seq_in, const Tensor& seq_out, const Tensor& signs,
+                   const Tensor& rv, const Tensor& seq_in, const Tensor& seq_out, const Tensor& seq_lengths,
+                   const Tensor& signs,
                    const Tensor& thresholds, const OptTensor& centroids, const OptTensor& gaussian,
                    const OptTensor& gaussian_t, bool ip, int64_t row0, int64_t capacity, int64_t bits,
                    int64_t value_group, int64_t max_leaving, int64_t max_fill, uintptr_t stream) {
@@ -319,7 +320,7 @@ OptTensor tq_store(const Tensor& k, const Tensor& v, const OptTensor& key_codes,
       row0 < 0 || row0 + k.size(0) > rk.size(0) || !plain(rk, dev) || !plain(rv, dev) || !rk.is_contiguous() ||
       !rv.is_contiguous())
     return std::nullopt;
-  for (const Tensor* t : {&seq_in, &seq_out, &signs, &thresholds})
+  for (const Tensor* t : {&seq_in, &seq_out, &seq_lengths, &signs, &thresholds})
     if (!plain(*t, dev) || !t->is_contiguous()) return std::nullopt;
   for (const OptTensor* t : {&key_codes, &key_norms, &key_signs, &key_residual_norms, &key_dense, &vdata, &vscales, &vzeros,
                              &centroids, &gaussian, &gaussian_t})
@@ -347,6 +348,7 @@ OptTensor tq_store(const Tensor& k, const Tensor& v, const OptTensor& key_codes,
   a.residual_key = ptr(rk), a.residual_value = ptr(rv);
   a.seq_in = (const int32_t*)ptr(seq_in);
   a.seq_out = (int32_t*)ptr(seq_out);
+  a.seq_lengths = (int32_t*)ptr(seq_lengths);
   a.past_out = (int64_t*)ptr(past);
   a.max_leaving = max_leaving, a.max_fill = max_fill;
   a.signs = (const float*)ptr(signs);

@@ -11,7 +11,8 @@
 // The launch has three kinds of 512-thread workgroups: tiles of keys, values, and ring fills.  A
 // ring slot is read and written by one wave only (its reading lanes are its writing lanes), so the
 // kinds need no order among them.  Lengths are read from one array and the new ones written to
-// another, so no workgroup can see a length another has already raised.
+// another, so no workgroup can see a length another has already raised; a third one, which stays the
+// same from launch to launch, is for the decode.
 //
 // What bounds it.  Inner-product keys: the two D x D fp32 products of a vector (4 D^2 flops) on the
 // matrix cores.  2 x 8064 leaving tokens of 2 KV heads, D = 256: 125 us, of which the products are
@@ -335,7 +336,11 @@ __global__ __launch_bounds__(ST_THREADS, TV > 16 ? 4 : 1) void tq_store_kernel(c
       const bool mine = b >= a.row0 && b < a.row0 + a.rows;
       const int L = a.seq_in ? a.seq_in[b] : 0;
       if (a.past_out) a.past_out[b] = L;
-      if (mine || a.seq_in) a.seq_out[b] = L + (mine ? (int)a.tokens : 0);
+      if (mine || a.seq_in) {
+        const int n = L + (mine ? (int)a.tokens : 0);
+        a.seq_out[b] = n;
+        if (a.seq_lengths) a.seq_lengths[b] = n;
+      }
     }
   }
   if (blockIdx.x < g.key_wgs) {
@@ -409,7 +414,8 @@ extern "C" int anna_mi_tq_store(const anna_mi_tq_store_args* ap, void* stream) {
   ANNA_CHECK(!ip || (a.centroids && a.gaussian && a.gaussian_t), "anna_mi_tq_store: null quantizer tables");
   ANNA_CHECK(!ip || a.max_leaving == 0 || (a.key_signs && a.key_residual_norms && a.key_dense),
              "anna_mi_tq_store: null key state");
-  ANNA_CHECK(a.seq_out != a.seq_in, "anna_mi_tq_store: the new lengths need an array of their own");
+  ANNA_CHECK(a.seq_out != a.seq_in && (!a.seq_lengths || a.seq_lengths != a.seq_in),
+             "anna_mi_tq_store: the new lengths need an array of their own");
   const int64_t es = a.dtype == ANNA_MI_F32 ? 4 : 2, per = 16 / es;
   auto aligned = [&](const void* p, int64_t s0, int64_t s1, int64_t s2) {
     return (uintptr_t)p % 16 == 0 && s0 % per == 0 && s1 % per == 0 && s2 % per == 0;

@@ -57,9 +57,10 @@ class _LayerSlab:
         self.value_group_size = value_group_size or _resolve_value_group_size(head_dim)
         self.capacity = 0
         self.lengths = [0] * batch
-        # device lengths: an append reads one array and writes the other, which becomes seq_lengths
+        # device lengths.  seq_lengths is one array for good: a captured decode holds its address.  The
+        # one-launch append reads one of the other two and writes the other and seq_lengths
         self.seq_lengths = torch.zeros((batch,), dtype=torch.int32, device=device)
-        self._next_lengths = torch.zeros_like(self.seq_lengths)
+        self._lengths_in, self._lengths_out = torch.zeros_like(self.seq_lengths), torch.zeros_like(self.seq_lengths)
         # one launch per append (anna_mi_tq_store) wherever the keys' rotation is the Hadamard one;
         # other head_dims (TQ-MSE keys, or no token past the window) go quantizer by quantizer
         self._qn = None
@@ -181,11 +182,12 @@ class _LayerSlab:
             (self.kidx, self.knorms, self.kqjl, self.krn, self.kdense) if ip else (self.kcodes, self.knorms, None, None, None))
         past = _lib.host().tq_store(
             keys, values, *key_state, *((self.vdata, self.vscales, self.vzeros) if C else (None,) * 3), self.rk, self.rv,
-            self.seq_lengths, self._next_lengths, qn.signs, qn.thresholds, *((qn.centroids, qn.gaussian, qn.gaussian_t)
-            if ip else (None,) * 3), ip, row0, C, self.bits, self.value_group_size, leaving, fill, _lib.stream_of(keys))
+            self._lengths_in, self._lengths_out, self.seq_lengths, qn.signs, qn.thresholds,
+            *((qn.centroids, qn.gaussian, qn.gaussian_t) if ip else (None,) * 3), ip, row0, C, self.bits,
+            self.value_group_size, leaving, fill, _lib.stream_of(keys))
         if past is None:
             raise RuntimeError("TurboQuant append: keys/values must be plain device tensors of the cache's dtype")
-        self.seq_lengths, self._next_lengths = self._next_lengths, self.seq_lengths
+        self._lengths_in, self._lengths_out = self._lengths_out, self._lengths_in
         return past
 
     def _append_step(self, keys: torch.Tensor, values: torch.Tensor) -> None:

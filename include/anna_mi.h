@@ -439,6 +439,8 @@ typedef struct {
   const float* gaussian_t;
   int value_lane_groups;       /* set by the library */
   float k0;                    /* set by the library */
+  int32_t* seq_lengths;        /* device [B]: receives what seq_out does, or NULL.  For a caller that alternates
+                                  seq_in and seq_out and whose readers want one array */
 } anna_mi_tq_store_args;
 
 int64_t anna_mi_sizeof_tq_store_args(void);

@@ -160,3 +160,36 @@ def test_pool_load_equals_appends(gpu, length, window):
     same(one.residual_value_t[..., :r], two.residual_value_t[..., :r])
     query = torch.randn(batch, 2 * heads, D, device=gpu, dtype=torch.bfloat16)
     same(one.decode(query, scaling=0.06), two.decode(query, scaling=0.06))
+
+
+@pytest.mark.parametrize("quantizer", ["ip", "mse"])
+def test_captured_decode_follows_the_appends(gpu, quantizer):
+    """A decode captured in a graph reads the lengths of the replay: tokens appended between replays count,
+    whether to every sequence or to one."""
+    torch.manual_seed(8)
+    head_dim = 128
+    cache = TurboQuantDynamicCache(1, kv_cache_residual_len=16, key_quantizer=quantizer)
+    new = lambda *s: torch.randn(*s, head_dim, device=gpu, dtype=torch.bfloat16)
+    k, v = new(2, 2, 40), new(2, 2, 40)
+    cache.update(k, v, 0, require_dense_cache=False)
+    k, v = new(2, 2, 1), new(2, 2, 1)
+    cache.update(k, v, 0, require_dense_cache=False)  # the slab has room from here on
+    q = new(2, 4, 1)
+    call = lambda: cache.turboquant_single_token_decode_attention(0, q, scaling=0.1, num_key_value_groups=2)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        call()
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    lengths = cache._slabs[0].seq_lengths
+    for step in range(5):
+        if step == 2:
+            cache.append_row(0, 1, *(new(2, 3) for _ in range(2)))
+        elif step:
+            cache.update(new(2, 2, 1), new(2, 2, 1), 0, require_dense_cache=False)
+        graph.replay()
+        same(out, call())
+        assert cache._slabs[0].seq_lengths is lengths and lengths.tolist() == cache.layer_lengths[0]
