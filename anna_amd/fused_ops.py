@@ -607,11 +607,14 @@ def tq_store_rows(tensor):
     16-byte aligned (a copy where they are not)."""
     per = 16 // tensor.element_size()
     s0, s1, s2, s3 = tensor.stride()
+    if s3 == 1 and not (s0 % per or s1 % per or s2 % per or tensor.data_ptr() % 16):
+        return tensor
+    # the stride of a single row, head or token is read by nobody and may be anything, also in a tensor
+    # that torch calls contiguous
+    s0, s1, s2 = (s if n > 1 else 0 for s, n in zip((s0, s1, s2), tensor.shape))
     if s3 != 1 or s0 % per or s1 % per or s2 % per or tensor.data_ptr() % 16:
-        tensor = tensor.contiguous()
-        if tensor.data_ptr() % 16:
-            tensor = tensor.clone()
-    return tensor
+        return tensor.clone(memory_format=torch.contiguous_format)
+    return tensor.as_strided(tensor.shape, (s0, s1, s2, 1))
 
 
 # ---------------------------------------------------------------- tiled int4 GEMV, LM-head top-k

@@ -193,3 +193,46 @@ def test_captured_decode_follows_the_appends(gpu, quantizer):
         graph.replay()
         same(out, call())
         assert cache._slabs[0].seq_lengths is lengths and lengths.tolist() == cache.layer_lengths[0]
+
+
+def odd_strides(t):
+    """t with a stride of 1 in each dimension of size 1: contiguous to torch, whose rule skips those"""
+    out = t.clone(memory_format=torch.contiguous_format)
+    return out.as_strided(t.shape, [1 if n == 1 else s for n, s in zip(t.shape, out.stride())])
+
+
+@pytest.mark.parametrize("batch,heads,tokens", [(3, 2, 1), (1, 2, 1), (1, 2, 40), (2, 1, 9), (1, 1, 1), (1, 1, 40)])
+@pytest.mark.parametrize("key_quantizer", ["ip", "mse"])
+def test_store_takes_any_stride_of_a_single_row(gpu, batch, heads, tokens, key_quantizer):
+    torch.manual_seed(tokens)
+    caches = [TurboQuantDynamicCache(1, kv_cache_residual_len=16, key_quantizer=key_quantizer) for _ in range(2)]
+    for n in (tokens, 20, tokens):
+        k, v = (torch.randn(batch, heads, n, 128, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        caches[0].update(k, v, 0, require_dense_cache=False)
+        caches[1].update(odd_strides(k), odd_strides(v), 0, require_dense_cache=False)
+    for (ak, av), (bk, bv) in zip(*([r.materialize() for r in c.turboquant_rows[0]] for c in caches)):
+        same(ak, bk)
+        same(av, bv)
+
+
+@pytest.mark.parametrize("head_dim,bits", [(128, 4)])
+@pytest.mark.parametrize("heads,length", [(2, 1), (1, 1), (1, 150), (2, 150)])
+def test_load_takes_any_stride_of_a_single_row(gpu, head_dim, bits, heads, length):
+    torch.manual_seed(length)
+    k, v = (torch.randn(heads, length, head_dim, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+    q = torch.randn(1, 2 * heads, head_dim, device=gpu, dtype=torch.bfloat16)
+    out = []
+    for a, b in ((k, v), (odd_strides(k), odd_strides(v)), (odd_strides(k), v), (k, odd_strides(v))):
+        cache = TurboQuantBatchCache(batch=1, kv_heads=heads, q_heads=2 * heads, capacities=[64], head_dim=head_dim,
+                                     bits=bits)
+        cache.load_sequence(0, a, b)
+        out.append(cache.decode(q, scaling=0.09))
+    for o in out[1:]:
+        same(o, out[0])
+    # a token stride that no row of 8 bytes fits, of one token: nothing is read at it
+    wide = torch.empty(heads * (head_dim + 1), device=gpu, dtype=torch.bfloat16)[:heads * head_dim]
+    one = wide.view(heads, 1, head_dim).as_strided((heads, 1, head_dim), (head_dim, head_dim + 1, 1)).copy_(k[:, :1])
+    cache.load_sequence(0, one, one)
+    first = cache.decode(q, scaling=0.09)
+    cache.load_sequence(0, k[:, :1], k[:, :1])
+    same(first, cache.decode(q, scaling=0.09))
