@@ -127,23 +127,27 @@ class TurboQuantBatchCache:
         """One launch: the first `tokens` tokens of keys/values [Hkv, L, D] into the pool, the newest
         ones into the ring, and the length."""
         _lib.require_device(keys, values, self.residual_key)
-        # the launch reads both with one set of strides, 8 bytes of a row at a time
-        if (keys.stride(2) != 1 or values.stride() != keys.stride() or keys.stride(0) % 4 or keys.stride(1) % 4
-                or keys.stride(1) < keys.shape[2] or keys.data_ptr() % 8 or values.data_ptr() % 8):
+        # the launch reads both with one set of strides, 8 bytes of a row at a time; the stride of a
+        # single head or token is read by nobody
+        H, L, D = keys.shape
+        head, token = (keys.stride(0) if H > 1 else 0), (keys.stride(1) if L > 1 else D)
+        if (keys.stride(2) != 1 or values.stride(2) != 1 or (H > 1 and values.stride(0) != head)
+                or (L > 1 and values.stride(1) != token) or head % 4 or token % 4 or token < D
+                or keys.data_ptr() % 8 or values.data_ptr() % 8):
             keys, values = (t.contiguous() if t.data_ptr() % 8 == 0 else t.clone(memory_format=torch.contiguous_format)
                             for t in (keys, values))
+            head, token = L * D, D
         a = _lib.TQLoadArgs()
         p = a.pack
         p.kv_heads, p.head_dim, p.tokens = self.kv_heads, self.head_dim, tokens
         p.keys, p.values = keys.data_ptr(), values.data_ptr()
-        p.stride_head = keys.stride(0) if self.kv_heads > 1 else 0
-        p.stride_token = max(keys.stride(1), self.head_dim)
+        p.stride_head, p.stride_token = head, token
         p.key_codes, p.key_norms = self.key_codes.data_ptr(), self.key_norms.data_ptr()
         p.value_codes, p.value_norms = self.value_codes.data_ptr(), self.value_norms.data_ptr()
         p.pool_tokens, p.slot_offset = self.pool_tokens, self.offsets[b]
         p.signs, p.thresholds = self.qn.signs.data_ptr(), self.qn.thresholds.data_ptr()
-        H, R, D = self.kv_heads, self.residual_capacity, self.head_dim
-        a.length, a.residual_capacity = keys.shape[1], R
+        R = self.residual_capacity
+        a.length, a.residual_capacity = L, R
         a.residual_key = self.residual_key.data_ptr() + 2 * b * H * R * D
         a.residual_value_t = self.residual_value_t.data_ptr() + 2 * b * H * R * D
         a.seq_length = self.seq_lengths.data_ptr() + 4 * b

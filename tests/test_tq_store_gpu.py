@@ -215,7 +215,7 @@ def test_store_takes_any_stride_of_a_single_row(gpu, batch, heads, tokens, key_q
         same(av, bv)
 
 
-@pytest.mark.parametrize("head_dim,bits", [(128, 4)])
+@pytest.mark.parametrize("head_dim,bits", [(128, 4), (256, 2)])
 @pytest.mark.parametrize("heads,length", [(2, 1), (1, 1), (1, 150), (2, 150)])
 def test_load_takes_any_stride_of_a_single_row(gpu, head_dim, bits, heads, length):
     torch.manual_seed(length)
