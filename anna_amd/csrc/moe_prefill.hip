@@ -509,6 +509,11 @@ bool pf_shape_ok(const anna_mi_moe_prefill_args& a) {
          a.intermediate_dim * a.hidden_packed_cols * 4 < lim && a.hidden_dim * a.intermediate_packed_cols * 4 < lim &&
          a.intermediate_dim * a.hidden_groups * 4 < lim && a.hidden_dim * a.intermediate_groups * 4 < lim;
 }
+// rows and words are read 16 bytes at a time
+bool pf_aligned(const anna_mi_moe_prefill_args& a) {
+  return a.hidden_row_stride % 8 == 0 && (uintptr_t)a.hidden % 16 == 0 && (uintptr_t)a.gate_qweight % 16 == 0 &&
+         (uintptr_t)a.up_qweight % 16 == 0 && (uintptr_t)a.down_qweight % 16 == 0;
+}
 
 }  // namespace
 }  // namespace anna
@@ -521,7 +526,7 @@ extern "C" int64_t anna_mi_sizeof_moe_prefill_args(void) { return (int64_t)sizeo
 // forms of moe.hip, 64 tokens of 32 experts, top 8 (16) 50 against 46, 128 experts, top 8: 64 tokens (4) 96
 // against 88, 128 tokens (8) 100 against 101, 512 tokens (32) 137 against 161, 2048 (128) 320 against 440.
 extern "C" int64_t anna_mi_moe_prefill_workspace(const anna_mi_moe_prefill_args* ap) {
-  if (!ap || !pf_shape_ok(*ap)) return 0;
+  if (!ap || !pf_shape_ok(*ap) || !pf_aligned(*ap)) return 0;
   if (ap->tokens * ap->top_k < 18 * ap->num_experts) return 0;
   return pf_layout(pf_plan(*ap)).total;
 }
@@ -534,11 +539,9 @@ extern "C" int anna_mi_moe_prefill(const anna_mi_moe_prefill_args* ap, void* str
   ANNA_CHECK(a.hidden && a.logits && a.out && a.workspace && a.slots && a.gate_qweight && a.gate_qscale && a.gate_qzeros &&
                  a.up_qweight && a.up_qscale && a.up_qzeros && a.down_qweight && a.down_qscale && a.down_qzeros,
              "anna_mi_moe_prefill: null pointer");
-  ANNA_CHECK(a.hidden_row_stride >= a.hidden_dim && a.hidden_row_stride % 8 == 0 && (uintptr_t)a.hidden % 16 == 0 &&
-                 (uintptr_t)a.out % 16 == 0 && (uintptr_t)a.workspace % 256 == 0,
-             "anna_mi_moe_prefill: rows must be 16-byte aligned, the workspace 256-byte aligned");
-  ANNA_CHECK((uintptr_t)a.gate_qweight % 16 == 0 && (uintptr_t)a.up_qweight % 16 == 0 && (uintptr_t)a.down_qweight % 16 == 0,
-             "anna_mi_moe_prefill: weights must be 16-byte aligned");
+  ANNA_CHECK(pf_aligned(a) && a.hidden_row_stride >= a.hidden_dim && (uintptr_t)a.out % 16 == 0 &&
+                 (uintptr_t)a.workspace % 256 == 0,
+             "anna_mi_moe_prefill: rows and weights must be 16-byte aligned, the workspace 256-byte aligned");
   ANNA_CHECK(a.logits_row_stride >= a.num_experts, "anna_mi_moe_prefill: bad logits stride");
   const PfPlan p = pf_plan(a);
   const PfLayout l = pf_layout(p);

@@ -393,7 +393,7 @@ OptTensor moe_block(const Tensor& x, const Tensor& logits, const Tensor& gq, con
   if (!is(experts, dev, at::kLong) || !is(slots, dev, at::kLong) || experts.numel() != E || slots.numel() != E)
     return std::nullopt;
   const int64_t I = gq.size(1);
-  if (x.stride(0) % 8 == 0 && (uintptr_t)ptr(x) % 16 == 0 && dq.size(1) == H && ds.size(2) == H && gs.size(2) == I) {
+  if (dq.size(1) == H && ds.size(2) == H && gs.size(2) == I) {
     anna_mi_moe_prefill_args p{};
     p.dtype = dt, p.logits_dtype = ldt, p.scale_dtype = sdt, p.normalize = normalize;
     p.tokens = T, p.num_experts = E, p.top_k = top_k, p.hidden_dim = H, p.intermediate_dim = I, p.group_size = group;

@@ -92,3 +92,18 @@ def test_prefill_block_one_expert_past_a_million_routes(gpu):
     got = block(x, logits)
     for a in range(0, tokens, 100_000):
         assert torch.equal(got[a:a + 100_000], block(x[a:a + 100_000], logits[a:a + 100_000]))
+
+
+def test_unaligned_bank_takes_the_general_way(gpu):
+    """Weights that are 4-byte aligned only (slices of one storage) give what aligned ones give."""
+    bank = make_bank(16, 256, 256, 128, torch.float32, gpu, 11)
+    torch.manual_seed(11)
+    x = torch.randn(200, 256, device=gpu, dtype=torch.bfloat16)
+    logits = torch.randn(200, 16, device=gpu)
+    ref = brute_force(bank, x, logits, 4, True)
+    for name in ("gate_qweight", "up_qweight", "down_qweight"):
+        w = getattr(bank, name)
+        room = torch.empty(w.numel() + 1, dtype=w.dtype, device=gpu)
+        setattr(bank, name, room[1:].view(w.shape).copy_(w))
+        got = SparseMoeInt4(bank, num_experts=16, top_k=4)(x, logits)
+        assert rel_err(got.double().cpu().numpy(), ref) <= BF16_TOL
