@@ -378,11 +378,14 @@ class XPUInt4Linear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.is_cuda:
+            # straight from where the constructor put them (attribute access costs four lookups); a tensor
+            # replaced or parametrized since is another place's: the general way asks for the attribute
             b, p = self._buffers, self._parameters
-            out = _lib.host().int4_linear(x, b["qweight"], b["qscale"], b["qzeros"], p["bias"], self.group_size,
-                                          self.out_features, self.compute_dtype, _lib.stream_of(x))
-            if out is not None:
-                return out
+            if "qweight" in b and "qscale" in b and "qzeros" in b and "bias" in p:
+                out = _lib.host().int4_linear(x, b["qweight"], b["qscale"], b["qzeros"], p["bias"], self.group_size,
+                                              self.out_features, self.compute_dtype, _lib.stream_of(x))
+                if out is not None:
+                    return out
         lead = x.shape[:-1]
         x2d = x.reshape(-1, x.shape[-1]).to(self.compute_dtype)
         _require_rocm(x2d, "XPUInt4Linear.forward")
