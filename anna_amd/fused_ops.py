@@ -128,7 +128,7 @@ def int4_linear_out(hidden_states, qweight, qscale, qzeros, group_size, in_featu
 
 
 def _xpu_int4_gemv_impl(hidden_states, qweight, qscale, qzeros, group_size, in_features):
-    if hidden_states.dim() == 2 and hidden_states.size(1) == in_features and qweight.dim() == 2:
+    if hidden_states.is_cuda and hidden_states.dim() == 2 and hidden_states.size(1) == in_features and qweight.dim() == 2:
         out = _lib.host().int4_linear(hidden_states, qweight, qscale, qzeros, None, group_size, qweight.size(0),
                                       hidden_states.dtype, _lib.stream_of(hidden_states), False)
         if out is not None:

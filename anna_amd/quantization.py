@@ -378,8 +378,8 @@ class XPUInt4Linear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.is_cuda:
-            # straight from where the constructor put them (attribute access costs four lookups); a tensor
-            # replaced or parametrized since is another place's: the general way asks for the attribute
+            # read where the constructor registered them, not through Module.__getattr__; a tensor that
+            # has been replaced or parametrized since is somewhere else, and the general way finds it
             b, p = self._buffers, self._parameters
             if "qweight" in b and "qscale" in b and "qzeros" in b and "bias" in p:
                 out = _lib.host().int4_linear(x, b["qweight"], b["qscale"], b["qzeros"], p["bias"], self.group_size,

@@ -111,3 +111,10 @@ def test_moe_combine_checks_route_pos():
         fused_ops.moe_combine(co, torch.zeros(6, dtype=torch.int64), 4, 2)
     with pytest.raises(RuntimeError, match="fewer compact rows"):
         fused_ops.moe_combine(co, torch.zeros(10, dtype=torch.int64), 5, 2)
+
+
+def test_int4_gemv_names_the_device_of_host_activations():
+    with pytest.raises(RuntimeError, match="need ROCm device tensors, got a tensor on cpu"):
+        fused_ops._xpu_int4_gemv_impl(torch.zeros(2, 256, dtype=torch.bfloat16),
+                                      torch.zeros(96, 32, dtype=torch.int32), torch.zeros(2, 96),
+                                      torch.zeros(2, 96, dtype=torch.int8), 128, 256)
