@@ -112,14 +112,14 @@ class TurboQuantBatchCache:
         q = max(0, L - R)
         if q > self.capacities[b]:
             raise ValueError(f"sequence {b}: {q} quantized tokens exceed its capacity {self.capacities[b]}")
-        if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
-            raise ValueError("keys/values must be bf16")
-        if D != self.head_dim:
-            raise ValueError(f"keys/values must have head_dim {self.head_dim}, got {D}")
         if L == 0:
             self.seq_lengths[b] = 0
         else:
-            k, v = keys.expand(self.kv_heads, L, D), values.expand(self.kv_heads, L, D)
+            if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
+                raise ValueError("keys/values must be bf16")
+            if q > 0 and D != self.head_dim:
+                raise ValueError(f"keys/values must have head_dim {self.head_dim}, got {D}")
+            k, v = (t.expand(self.kv_heads, L, self.head_dim) for t in (keys, values))
             self._load(range(self.batch)[b], k, v, q)
         self.lengths[b] = L
 
@@ -330,12 +330,12 @@ class TurboQuantRowsCache(TurboQuantBatchCache):
             raise ValueError(f"sequence {b}: {q} quantized tokens exceed its capacity {self.capacities[b]}")
         if keys.dtype != torch.bfloat16 or values.dtype != torch.bfloat16:
             raise ValueError("keys/values must be bf16")
-        if D != self.head_dim:
-            raise ValueError(f"keys/values must have head_dim {self.head_dim}, got {D}")
         if L == 0:
             self.seq_lengths[b] = 0
         else:
-            self._store(range(self.batch)[b], keys.expand(self.kv_heads, L, D), values.expand(self.kv_heads, L, D))
+            if q > 0 and D != self.head_dim:
+                raise ValueError(f"keys/values must have head_dim {self.head_dim}, got {D}")
+            self._store(range(self.batch)[b], *(t.expand(self.kv_heads, L, self.head_dim) for t in (keys, values)))
         self.lengths[b] = L
 
     def _store(self, b: int, keys: torch.Tensor, values: torch.Tensor) -> None:

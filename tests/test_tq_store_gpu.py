@@ -236,3 +236,26 @@ def test_load_takes_any_stride_of_a_single_row(gpu, head_dim, bits, heads, lengt
     first = cache.decode(q, scaling=0.09)
     cache.load_sequence(0, k[:, :1], k[:, :1])
     same(first, cache.decode(q, scaling=0.09))
+
+
+def test_load_of_nothing_and_of_other_types(gpu):
+    """No tokens: any head_dim, and in the 2-bit pool any type, as there is nothing to read."""
+    for head_dim, bits in ((256, 2), (128, 4)):
+        cache = TurboQuantBatchCache(batch=1, kv_heads=2, q_heads=4, capacities=[64], head_dim=head_dim, bits=bits)
+        k = torch.randn(2, 5, head_dim, device=gpu, dtype=torch.bfloat16)
+        cache.load_sequence(0, k, k)
+        if bits == 2:
+            cache.load_sequence(0, k[:, :0].float(), k[:, :0].float())
+        cache.load_sequence(0, k[:, :0, :64], k[:, :0, :64])
+        assert cache.lengths == [0] == cache.seq_lengths.tolist()
+        long = torch.randn(2, 150, head_dim, device=gpu, dtype=torch.bfloat16)
+        for bad in (k.float(), k[..., :64], long[..., :64], long[..., :1]):
+            with pytest.raises((ValueError, RuntimeError)):
+                cache.load_sequence(0, bad, bad)
+        # within the window a head, a token or a dimension of size 1 stands for all of them
+        q = torch.randn(1, 4, head_dim, device=gpu, dtype=torch.bfloat16)
+        for part in (k[:1], k[..., :1]):
+            cache.load_sequence(0, part, part)
+            got = cache.decode(q, scaling=0.09)
+            cache.load_sequence(0, part.expand_as(k).contiguous(), part.expand_as(k).contiguous())
+            same(got, cache.decode(q, scaling=0.09))
