@@ -394,7 +394,8 @@ extern "C" int anna_mi_tq_store(const anna_mi_tq_store_args* ap, void* stream) {
              "anna_mi_tq_store: head_dim must be a power of two in [64, 1024]");
   ANNA_CHECK(a.key_bits >= (ip ? 2 : 1) && a.key_bits <= 4, "anna_mi_tq_store: bad key bits");
   ANNA_CHECK(a.value_bits >= 2 && a.value_bits <= 4, "anna_mi_tq_store: value bits must be 2..4");
-  ANNA_CHECK(a.value_group_size > 0 && D % a.value_group_size == 0,
+  // (no values are grouped while nothing leaves the window)
+  ANNA_CHECK(a.max_leaving == 0 || (a.value_group_size > 0 && D % a.value_group_size == 0),
              "anna_mi_tq_store: value_group_size must divide head_dim");
   ANNA_CHECK(a.batch > 0 && a.kv_heads > 0 && a.rows > 0 && a.row0 >= 0 && a.row0 + a.rows <= a.batch,
              "anna_mi_tq_store: bad row range");

@@ -259,3 +259,14 @@ def test_load_of_nothing_and_of_other_types(gpu):
             got = cache.decode(q, scaling=0.09)
             cache.load_sequence(0, part.expand_as(k).contiguous(), part.expand_as(k).contiguous())
             same(got, cache.decode(q, scaling=0.09))
+
+
+def test_value_groups_matter_once_tokens_leave(gpu):
+    """A group size that does not divide head_dim is refused where a token is quantized, not before."""
+    cache = TurboQuantDynamicCache(1, kv_cache_residual_len=16, value_group_size=48)
+    k = torch.randn(2, 2, 16, 128, device=gpu, dtype=torch.bfloat16)
+    keys, values, _ = cache.update(k, k, 0)
+    same(keys, k)
+    same(values, k)
+    with pytest.raises((ValueError, RuntimeError)):
+        cache.update(k, k, 0)
