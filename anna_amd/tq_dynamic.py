@@ -161,6 +161,8 @@ class _LayerSlab:
                 for i in range(rows):
                     self._append_row(row0 + i, keys[i], values[i])
             self.seq_lengths[row0:row0 + rows] += T
+        elif rows == 0:
+            past = self.seq_lengths.long()
         else:
             past = self._store(row0, keys, values)
         for b in range(row0, row0 + rows):

@@ -270,3 +270,10 @@ def test_value_groups_matter_once_tokens_leave(gpu):
     same(values, k)
     with pytest.raises((ValueError, RuntimeError)):
         cache.update(k, k, 0)
+
+
+def test_update_of_no_sequences(gpu):
+    cache = TurboQuantDynamicCache(1, kv_cache_residual_len=16)
+    k = torch.randn(0, 2, 20, 128, device=gpu, dtype=torch.bfloat16)
+    _, _, past = cache.update(k, k, 0, require_dense_cache=False)
+    assert past.numel() == 0
