@@ -1007,6 +1007,21 @@ int launch_head_mfma(const void* x, int64_t M, int64_t K, int64_t xs, const uint
   return ANNA_MI_OK;
 }
 
+// Where the dot2 forms stay faster for a few rows of x.  They give a workgroup 16 rows of W and a row of x its
+// own pass of products; the MFMA form gives a workgroup 64 and computes up to 16 rows of x at the price of one,
+// in passes of 16 128-k blocks per workgroup, whole ones also where K leaves some of a pass idle.  us, dot2 and
+// MFMA (bf16): K = 512 (12 of 16 blocks idle) M = 1, N = 1000 3.4 and 5.6, M = 4, N = 4096 4.8 and 5.9, M = 2,
+// N = 24576 7.0 and 8.0, but M = 4, N = 12288 6.4 and 6.0; K = 2048 M = 1, N = 4096 4.4 and 6.2, M = 2 5.4 and
+// 6.3, but M = 3 6.5 and 6.4; K = 4096 M = 1, N = 24576 14.0 and 15.6, M = 3, N = 1000 8.8 and 9.2, but M = 2,
+// N = 12288 12.5 and 10.8;
+// K = 8192 M = 1, N = 8192 15.8 and 17.2, but N = 12288 20.1 and 17.3.
+bool tiled_dot2_faster(int64_t M, int64_t N, int64_t K) {
+  const int64_t blocks = K / 128, idle = (blocks + 15) / 16 * 16 - blocks;
+  if (K > 4096) return M <= 2 && M * M * N <= 8192;
+  if (K >= 512 && idle >= 8) return M <= (idle >= 12 ? 5 : 4) && N <= 32768 && M * M * N <= 98304;
+  return M <= (K < 512 ? 4 : K > 2048 ? 3 : 2) && M * M * N <= 24576;
+}
+
 // ANNA_MI_TILED_PLAIN=1 keeps the tiled GEMV off its LDS-staged form (for comparisons and tests)
 static const int g_tiled_plain = [] {
   const char* v = getenv("ANNA_MI_TILED_PLAIN");
@@ -1022,7 +1037,7 @@ int launch_tiled(const void* x, int64_t M, int64_t K, int64_t xs, const uint32_t
   // 40.0 against 42.7 us for one row (V = 151936, K = 2048), 42.5 against 104.9 for four, 92 against
   // 452 for sixteen
   if constexpr (XDT != ANNA_MI_F32) {
-    if (head_mfma_ok<XDT>(x, M, K, xs, qw, T, gsz) && !g_tiled_plain)
+    if (head_mfma_ok<XDT>(x, M, K, xs, qw, T, gsz) && !tiled_dot2_faster(M, N, K) && !g_tiled_plain)
       return launch_head_mfma<XDT, SDT, OUT_F32>(x, M, K, xs, qw, tiles, pc, qs, qz, ssg, ssn, gsz, N, y, ys, nullptr,
                                                  nullptr, st);
   }

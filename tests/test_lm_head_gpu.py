@@ -185,3 +185,26 @@ def test_lm_head_block_selection(gpu, k, n, rows, top_k, dtype, group):
     y = fused_ops.int4_gemv_tiled(x, q.lm_head_qweight, q.qscale.view(-1, n // 4, 4), q.qzeros.view(-1, n // 4, 4),
                                   group, k, n)
     assert rel_err(y.double().cpu().numpy(), ref.cpu().numpy()) <= BF16_TOL
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 24576, 128), (1, 24580, 128), (4, 1536, 256), (4, 1540, 256), (5, 300, 256),
+                                   (5, 3932, 512), (5, 3936, 512), (1, 32768, 512), (1, 32772, 512), (6, 300, 512),
+                                   (4, 6144, 768), (4, 6148, 768), (5, 300, 768), (2, 6144, 1152), (2, 6148, 1536),
+                                   (3, 300, 2048), (3, 2728, 4096), (3, 2732, 4096), (2, 2048, 4224), (2, 2052, 4224), (3, 300, 4224)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tiled_gemv_on_both_sides_of_its_forms(gpu, m, n, k, dtype):
+    """Tiles of 4 rows and whole 128-k blocks: the dot2 forms for few rows, the MFMA form beyond."""
+    g = torch.Generator(device=gpu).manual_seed(m * n + k)
+    qw = torch.randint(-(2**31), 2**31, (n // 4, k // 8, 4), dtype=torch.int32, device=gpu, generator=g)
+    qs = torch.rand(k // 128, n // 4, 4, device=gpu, generator=g) * 0.01 + 0.001
+    qz = torch.randint(0, 16, (k // 128, n // 4, 4), dtype=torch.int8, device=gpu, generator=g)
+    x = torch.randn(m, k, device=gpu, generator=g).to(dtype)
+    y = fused_ops.int4_gemv_tiled(x, qw, qs, qz, 128, k, n)
+    codes = torch.stack([(qw >> (4 * j)) & 15 for j in range(8)], dim=2).permute(0, 3, 1, 2).reshape(n, k)
+    zeros, scales = (t.reshape(k // 128, n).t().repeat_interleave(128, dim=1).double() for t in (qz, qs))
+    ref = x.double() @ ((codes - zeros) * scales).t()
+    # half a unit of the result's last place, and fp32 sums of x (128 + code) and x (128 + zero), no more than
+    # 128 roundings one after the other in either
+    bound = ref.abs() * (2.0**-8 if dtype == torch.bfloat16 else 2.0**-11) + \
+        (x.double().abs() @ scales.t()) * 2 * 143 * 128 * 2.0**-24
+    assert bool(((y.double() - ref).abs() <= bound).all())
