@@ -223,10 +223,11 @@ int int4_rows_launch(const void* x, int x_dtype, int64_t M, int64_t K, int64_t x
     using T2 = std::integral_constant<int, 2>;
     using T4 = std::integral_constant<int, 4>;
     auto go_mg = [&](auto xdt_tag, auto al_tag) {
-      // one row group up to 16 rows, with one tile of W a workgroup while that is no more than two
-      // workgroups a compute unit; two tiles beyond, and two or four row groups for more rows (the
+      // one row group and one tile of W a workgroup while that is no more than two workgroups a compute
+      // unit (K = 4095, N = 64, M = 64: 25 us; 84 in two workgroups of four groups, 67 with the scalar
+      // kernel; N = 1024 21.6, 75 and 132); two tiles beyond, and two or four row groups for more rows (the
       // conversion is shared by them: M = 48, K = 4096, N = 6144 20.7 us against three times 13)
-      if (M <= 16 && (N + 15) / 16 <= 512) go(xdt_tag, T1{}, T1{}, al_tag);
+      if (((N + 15) / 16) * ((M + 15) / 16) <= 512) go(xdt_tag, T1{}, T1{}, al_tag);
       else if (M <= 16) go(xdt_tag, T2{}, T1{}, al_tag);
       else if (M <= 32) go(xdt_tag, T2{}, T2{}, al_tag);
       else go(xdt_tag, T2{}, T4{}, al_tag);

@@ -39,6 +39,14 @@ CASES = [
     (40, 1001, 48, 32, 3, torch.float32),     # odd K and row stride
     (200, 129, 20, 64, 0, torch.float32),
     (2, 1, 5, 128, 0, torch.float32),         # the smallest K
+    # more than 512 pairs of a 16-row tile of W and a 16-row group of x: two tiles a workgroup
+    (16, 320, 8200, 32, 0, torch.float32),
+    (17, 640, 4113, 32, 0, torch.float32),    # and two row groups
+    (33, 1120, 2801, 32, 0, torch.bfloat16),  # four row groups, the last empty
+    (130, 1056, 930, 64, 0, torch.float32),   # three workgroups of rows
+    (70, 232, 1700, 64, 0, torch.float32),    # group 64 with K no multiple of 64
+    (40, 1001, 2800, 32, 3, torch.float32),   # odd K and row stride
+    (200, 129, 640, 128, 0, torch.float16),
 ]
 
 
