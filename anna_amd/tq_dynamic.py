@@ -452,6 +452,10 @@ class TurboQuantDynamicCache:
         B, H, T, D = key_states.shape
         self._ensure_batch_size(B)
         _require_rocm(key_states, "TurboQuantDynamicCache")
+        if torch.cuda.is_current_stream_capturing():
+            # the lengths are counted on the host and the append alternates between two device arrays:
+            # a replay would write the captured step's slots again
+            raise RuntimeError("TurboQuantDynamicCache.update cannot be captured in a graph")
         slab = self._slabs[layer_idx]
         if slab is None:
             slab = _LayerSlab(batch=B, heads=H, head_dim=D, dtype=key_states.dtype, device=key_states.device,

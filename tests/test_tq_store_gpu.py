@@ -277,3 +277,19 @@ def test_update_of_no_sequences(gpu):
     k = torch.randn(0, 2, 20, 128, device=gpu, dtype=torch.bfloat16)
     _, _, past = cache.update(k, k, 0, require_dense_cache=False)
     assert past.numel() == 0
+
+
+def test_update_is_refused_in_a_capture(gpu):
+    """The host counts the lengths and the append's arrays alternate, so that a replay would store the
+    captured step again; a refused update leaves the cache as it was."""
+    cache = TurboQuantDynamicCache(1, kv_cache_residual_len=16)
+    k = torch.randn(2, 2, 20, 128, device=gpu, dtype=torch.bfloat16)
+    cache.update(k, k, 0, require_dense_cache=False)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        one = k[:, :, :1] + 0
+        with pytest.raises(RuntimeError, match="captured"):
+            cache.update(one, one, 0, require_dense_cache=False)
+    assert cache.layer_lengths == [[20, 20]]
+    cache.update(k[:, :, :1], k[:, :, :1], 0, require_dense_cache=False)
+    assert cache._slabs[0].seq_lengths.tolist() == [21, 21]
