@@ -26,6 +26,8 @@
 // 445 -> 320; 32 experts of 768 1060 -> 345.  Measured and not kept: 8 waves of two operands against
 // up to 128 routes in one workgroup per compute unit (181 + 140 us; W is converted once, but nothing fills
 // the barriers).
+#include <stdlib.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -522,12 +524,33 @@ using namespace anna;
 
 extern "C" int64_t anna_mi_sizeof_moe_prefill_args(void) { return (int64_t)sizeof(anna_mi_moe_prefill_args); }
 
-// From 18 routes per expert on average: 300 tokens of 64 experts, top 4 (18.75) 51 against 54 us with the
-// forms of moe.hip, 64 tokens of 32 experts, top 8 (16) 50 against 46, 128 experts, top 8: 64 tokens (4) 96
-// against 88, 128 tokens (8) 100 against 101, 512 tokens (32) 137 against 161, 2048 (128) 320 against 440.
+// Where this form is faster than those of moe.hip (us, this form and those; 738 shapes of 4 to 128 experts, hidden
+// 512 to 4096, intermediate 256 to 4096, 18 to 128 routes per expert: 0.3% from the better one on average, and at
+// most 12% slower than those where it is taken).  Never below 18 routes per expert (64 tokens of 32 experts, top 8 (16) 50 and 46); above:
+//  - where moe.hip has its wide and resident forms (intermediate 256 or 512, hidden a multiple of 256): from
+//    1024 x 512 on (128 experts of 2048 x 512, top 8, 18 routes 95 and 108, 64 302 and 440); narrower ones keep this
+//    form's five launches too short of work until there are 36 routes or many tokens (16 experts of 512 x 256, 24
+//    routes 45 and 39, 48 46 and 52; 32 of 2048 x 256, top 8, 96 tokens 70 and 64; 64 of 1024 x 256, top 2, 1024
+//    tokens 60 and 68);
+//  - else, where the 16-route kernels are the other form, by the work and the sweeps those need: 8 experts of
+//    512 x 768, 24 routes 55 and 39, 64 55 and 56; 64 of 1024 x 768, 18 routes 59 and 81; 16 of 1024 x 768, 24
+//    routes 48 and 43, 16 of 2048 x 1408 59 and 79.
+static bool pf_faster(int64_t tokens, int64_t experts, int64_t top_k, int64_t hidden, int64_t inter) {
+  const int64_t routes = tokens * top_k;
+  if (routes < 18 * experts) return false;
+  if (inter % 256 == 0 && inter <= 512 && hidden % 256 == 0)
+    return (hidden >= 1024 && inter >= 512) || routes >= 36 * experts || tokens * hidden * inter >= 1ll << 27;
+  return routes >= 64 * experts || (double)routes * routes / experts * hidden * inter >= 8589934592.0;
+}
+
 extern "C" int64_t anna_mi_moe_prefill_workspace(const anna_mi_moe_prefill_args* ap) {
   if (!ap || !pf_shape_ok(*ap) || !pf_aligned(*ap)) return 0;
-  if (ap->tokens * ap->top_k < 18 * ap->num_experts) return 0;
+  // ANNA_MI_MOE_FORM = P forces this form, anything else the ones of moe.hip (read on every call; the tests run
+  // both on shapes small enough for the CPU oracle)
+  const char* f = getenv("ANNA_MI_MOE_FORM");
+  const bool take = f && *f ? f[0] == 'P'
+                            : pf_faster(ap->tokens, ap->num_experts, ap->top_k, ap->hidden_dim, ap->intermediate_dim);
+  if (!take) return 0;
   return pf_layout(pf_plan(*ap)).total;
 }
 

@@ -40,7 +40,7 @@ def test_router_rows_without_a_softmax(gpu, experts, top_k, dtype):
 
 
 # the routing in one launch, the separate router and dispatch, and the form for many routes per expert
-@pytest.mark.parametrize("tokens,experts,top_k", [(9, 16, 4), (60, 64, 4), (75, 16, 4)])
+@pytest.mark.parametrize("tokens,experts,top_k", [(9, 16, 4), (60, 64, 4), (75, 16, 4), (150, 16, 4)])
 def test_block_keeps_the_other_tokens(gpu, tokens, experts, top_k):
     torch.manual_seed(tokens)
     bank = make_bank(experts, 256, 256, 128, torch.float32, gpu, tokens)

@@ -6,7 +6,6 @@ import torch
 
 from anna_amd import _lib
 from anna_amd.moe import SparseMoeInt4
-from oracle import cpu_paths as cp
 from tests._util import BF16_TOL, rel_err
 from tests.test_moe_gpu import dequant_experts, make_bank
 
@@ -14,7 +13,10 @@ pytestmark = pytest.mark.gpu
 
 
 def brute_force(bank, x, logits, top_k, norm):
-    w, sel, _ = cp.moe_route(logits.cpu(), top_k, norm)
+    # (as cp.moe_route, with equal logits in the order of their experts: 16-bit ones have some)
+    w, sel = (t[:, :top_k] for t in torch.softmax(logits.cpu(), dim=-1, dtype=torch.float32).sort(
+        dim=-1, descending=True, stable=True))
+    w = w / w.sum(dim=-1, keepdim=True) if norm else w
     out = torch.zeros(x.shape, dtype=torch.float64)
     experts = dequant_experts(bank, sorted(set(sel.reshape(-1).tolist())))
     xd = x.cpu().double()
@@ -25,7 +27,33 @@ def brute_force(bank, x, logits, top_k, norm):
     return out.numpy()
 
 
-# tokens x top_k / experts from 18 up: sweeps of one to three chunks, several sweeps, a ragged last tile
+# fp16 states: the activation between the products is rounded to bf16 (2^-9 of each element at most, so
+# 1.1e-3 of a sum of many in 2-norm; 1.7e-3 measured with the other roundings); the largest error over the
+# largest value is allowed about twice that
+FP16_TOL = 4e-3
+
+
+def takes_prefill(bank, x, logits, top_k):
+    """Whether the dispatch rule sends the call to the form tested here."""
+    a = _lib.MoePrefillArgs()
+    a.dtype, a.logits_dtype, a.scale_dtype = (_lib.dtype_code(t.dtype) for t in (x, logits, bank.gate_qscale))
+    a.tokens, a.num_experts, a.top_k, a.group_size = x.shape[0], logits.shape[1], top_k, bank.group_size
+    a.hidden_dim, a.intermediate_dim = bank.hidden_dim, bank.intermediate_dim
+    a.hidden, a.hidden_row_stride = x.data_ptr(), x.stride(0)
+    a.gate_qweight, a.up_qweight, a.down_qweight = (t.data_ptr() for t in (bank.gate_qweight, bank.up_qweight,
+                                                                         bank.down_qweight))
+    a.hidden_packed_cols, a.hidden_groups = bank.gate_qweight.shape[2], bank.gate_qscale.shape[1]
+    a.intermediate_packed_cols, a.intermediate_groups = bank.down_qweight.shape[2], bank.down_qscale.shape[1]
+    return _lib.load().anna_mi_moe_prefill_workspace(a) > 0
+
+
+@pytest.fixture
+def forced(monkeypatch):
+    """The form on every shape it can compute, faster there or not."""
+    monkeypatch.setenv("ANNA_MI_MOE_FORM", "P")
+
+
+# sweeps of one to three chunks, several sweeps, a ragged last tile
 # (intermediate 384 = 3 x 128, hidden 384 = 1.5 x 256), one group of K, the most groups of K, one
 # token per wave and several, tokens past one workgroup's share
 @pytest.mark.parametrize("tokens,experts,top_k,hidden,inter,dtype,scales,norm", [
@@ -38,17 +66,18 @@ def brute_force(bank, x, logits, top_k, norm):
     (5003, 3, 1, 128, 128, torch.bfloat16, torch.float32, True),
     (40, 64, 64, 256, 128, torch.bfloat16, torch.float32, False),
 ])
-def test_prefill_block_matches_brute_force(gpu, tokens, experts, top_k, hidden, inter, dtype, scales, norm):
+def test_prefill_block_matches_brute_force(gpu, forced, tokens, experts, top_k, hidden, inter, dtype, scales, norm):
     bank = make_bank(experts, hidden, inter, 128, scales, gpu, tokens)
     torch.manual_seed(tokens)
     wide = torch.randn(tokens, hidden + 64, device=gpu).to(dtype)
     x = wide[:, :hidden]  # rows a stride apart
     logits = torch.randn(tokens, experts, device=gpu)
     block = SparseMoeInt4(bank, num_experts=experts, top_k=top_k, norm_topk_prob=norm)
-    ref = brute_force(bank, x, logits, top_k, norm)
-    assert rel_err(block(x, logits).double().cpu().numpy(), ref) <= BF16_TOL
-    # the reference's own 16-bit logits
-    block(x, logits.to(dtype))
+    tol = BF16_TOL if dtype == torch.bfloat16 else FP16_TOL
+    for lg in (logits, logits.to(dtype)):  # (16 bits: the reference's own logits)
+        assert takes_prefill(bank, x, lg, top_k)
+        ref = brute_force(bank, x, lg, top_k, norm)
+        assert rel_err(block(x, lg).double().cpu().numpy(), ref) <= tol
 
 
 def test_prefill_block_skewed_experts(gpu):
@@ -63,20 +92,29 @@ def test_prefill_block_skewed_experts(gpu):
     logits[:, 9] = 4.0 + torch.rand(tokens, device=gpu) * 0.5
     logits[17, 12] = 9.0
     block = SparseMoeInt4(bank, num_experts=experts, top_k=2)
+    assert takes_prefill(bank, x, logits, 2)
     got = block(x, logits)
     assert rel_err(got.double().cpu().numpy(), brute_force(bank, x, logits, 2, True)) <= BF16_TOL
     assert torch.equal(got, block(x, logits))  # no atomics: the same bits again
 
 
 def test_prefill_takes_only_its_shapes(gpu):
-    """Group 64, fp32 hidden states, dims off 128 and few routes go the general way."""
+    """Group 64, fp32 hidden states and rows that are not 16-byte aligned go the general way, and so do shapes
+    on which it is the faster one: both sides of each line of the rule."""
     torch.manual_seed(2)
-    for experts, hidden, inter, group, dtype, tokens in ((8, 256, 256, 64, torch.bfloat16, 64),
-                                                         (8, 256, 256, 128, torch.float32, 64),
-                                                         (32, 256, 256, 128, torch.bfloat16, 20)):
+    for experts, hidden, inter, group, dtype, tokens, pad, takes in (
+            (8, 256, 256, 64, torch.bfloat16, 300, 0, False), (8, 256, 256, 128, torch.float32, 300, 0, False),
+            (8, 256, 256, 128, torch.bfloat16, 300, 4, False), (8, 256, 256, 128, torch.bfloat16, 300, 0, True),
+            (32, 256, 256, 128, torch.bfloat16, 20, 0, False),
+            (8, 256, 256, 128, torch.bfloat16, 143, 0, False), (8, 256, 256, 128, torch.bfloat16, 144, 0, True),
+            (4, 1024, 512, 128, torch.bfloat16, 35, 0, False), (4, 1024, 512, 128, torch.bfloat16, 36, 0, True),
+            (64, 1024, 256, 128, torch.bfloat16, 511, 0, False), (64, 512, 256, 128, torch.bfloat16, 1024, 0, True),
+            (8, 384, 384, 128, torch.bfloat16, 255, 0, False), (8, 384, 384, 128, torch.bfloat16, 256, 0, True),
+            (4, 1024, 640, 128, torch.bfloat16, 114, 0, False), (4, 1024, 640, 128, torch.bfloat16, 115, 0, True)):
         bank = make_bank(experts, hidden, inter, group, torch.float32, gpu, 3)
-        x = torch.randn(tokens, hidden, device=gpu).to(dtype)
+        x = torch.randn(tokens, hidden + pad, device=gpu).to(dtype)[:, :hidden]
         logits = torch.randn(tokens, experts, device=gpu)
+        assert takes_prefill(bank, x, logits, 2) == takes
         block = SparseMoeInt4(bank, num_experts=experts, top_k=2)
         assert rel_err(block(x, logits).double().cpu().numpy(), brute_force(bank, x, logits, 2, True)) <= BF16_TOL
 
@@ -105,5 +143,6 @@ def test_unaligned_bank_takes_the_general_way(gpu):
         w = getattr(bank, name)
         room = torch.empty(w.numel() + 1, dtype=w.dtype, device=gpu)
         setattr(bank, name, room[1:].view(w.shape).copy_(w))
+        assert not takes_prefill(bank, x, logits, 4)
         got = SparseMoeInt4(bank, num_experts=16, top_k=4)(x, logits)
         assert rel_err(got.double().cpu().numpy(), ref) <= BF16_TOL
