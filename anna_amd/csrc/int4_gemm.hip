@@ -641,9 +641,10 @@ int int4_gemm_tiled_launch(const void* x, int x_dtype, int64_t M, int64_t K, int
   const bool msplit = tiles(TileM{}) <= 256 && (K / GM_BK) % (2 * TileM2::SPB) == 0;
   // Two small-tile workgroups share a compute unit, so that up to 512 of their tiles run in one round;
   // past that, and below a round of middle tiles, the middle tile with K split is faster.  M = 333:
-  // K = 4096, N = 6144 (768 small tiles) 52.0 -> 38.3 us, K = 1024, N = 4096 (516) 16.9 -> 14.3; M = 1000,
-  // K = N = 2048 (688) 26.9 -> 22.2; with no more than 512 the small tile stays: M = 257, K = 1024,
-  // N = 4096 (430) 11.9 against 14.2 us, M = 700, K = N = 2048 (473) 18.3 against 21.2.
+  // K = 4096, N = 6144 (768 small tiles) 53.2 -> 39.7 us, K = 1024, N = 4096 (516) 16.3 -> 13.9; M = 1000,
+  // K = N = 2048 (688) 28.2 -> 22.5; M = 128, K = 4096, N = 24576 66.6 -> 42.4; M = 65, N = 17408 51.1 -> 38.4
+  // (92 shapes of M = 65 to 500, K = 512 to 4096: none slower).  With no more than 512 the small tile stays:
+  // M = 257, K = 1024, N = 4096 (430) 11.1 against 13.7 us, M = 700, K = N = 2048 (473) 19.6 against 22.1.
   if (shape == 2 && msplit && tiles(TileS{}) > 512) shape = 1;
   // ANNA_MI_INT4_GEMM_TILE = L / M / S forces a tile shape (read on every call; the tests run
   // every shape on shapes small enough for the CPU oracle)

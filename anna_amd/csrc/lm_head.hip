@@ -12,13 +12,17 @@
 //                           (s * (sum x q - z sum x) per word), wave reduction at the end.
 //   int4_gemv_tiled_lds_kernel  (1..4 rows) the same with x and the tile scales and zero points
 //                           staged in LDS: one memory load per weight word.
+//   int4_head_mfma_kernel   T = 4, 16-bit x, whole 128-k blocks: 64 rows of W a workgroup against up to 16
+//                           rows of x on the matrix cores; with a selection to follow, also the best
+//                           logit of its 64.
+//   topk_blocks_kernel      that selection: the k best blocks of 64, then the k best of their logits.
 //   topk_rows_kernel        k <= 8, per row, 1024 threads: pass 1 takes each thread's maximum and
 //                           merges the maxima into a top-k list; its k-th entry bounds the row's
 //                           k-th best from below.  Pass 2 keeps only the logits at or above that
 //                           bound in sorted register lists, merged pairwise through LDS by a
 //                           bitonic merge (value descending, ties to the lower index).
 //   topk_rows_lds_kernel    k > 8: the same bound, the sorted lists in LDS.
-//   topk_chunk_wave_kernel, topk_merge_waves_kernel   k <= 8, few long rows (the fused LM head):
+//   topk_chunk_wave_kernel, topk_merge_waves_kernel   k <= 8, few long rows (the LM head's other forms):
 //                           one wave per 1024 logits keeps register lists whose heads a
 //                           tournament across the lanes pops in order; one wave per row merges
 //                           the chunk lists the same way.

@@ -22,8 +22,9 @@
 // LDS from the start.  The scale and zero point are applied per group in fp32 as
 // s (sum x (off + q) - (off + z) sum x); the activation between the products is bf16, as in the other
 // forms (moe.hip).  What bounds it: issue, ~6.5 VALU instructions (conversion, scaling, addresses) to an
-// MFMA.  2048 tokens, 128 experts, top 8, 2048 x 512: gate/up 203 -> 161 us, down 109 -> 107, the block
-// 445 -> 320; 32 experts of 768 1060 -> 345.  Measured and not kept: 8 waves of two operands against
+// MFMA.  2048 tokens, 128 experts, top 8, 2048 x 512, traced: gate/up 152 us, down 98, gather 33, route 15,
+// combine 13; the block with fp32 scales 289 to 307 us, with the forms of moe.hip 429 to 439; 32 experts of 768
+// 318 and 1077.  Measured and not kept: 8 waves of two operands against
 // up to 128 routes in one workgroup per compute unit (181 + 140 us; W is converted once, but nothing fills
 // the barriers).
 #include <stdlib.h>
@@ -594,8 +595,9 @@ extern "C" int anna_mi_moe_prefill(const anna_mi_moe_prefill_args* ap, void* str
     g.sweeps = (int)std::max<int64_t>(1, (p.routes * 3 / 2 / a.num_experts + 16 * PF_NC - 1) / (16 * PF_NC));
     auto launch = [&](auto gu_tag) {
       constexpr bool GU = decltype(gu_tag)::value;
-      // an item's steps fill the pipeline once: eight of them or more (the down product at K = 512: 132 us
-      // with 4 steps, 113 with 8, 107 with 16, which loses where items are few: 372 against 345 us a block)
+      // an item's steps fill the pipeline once: eight of them or more (the down product at K = 512, with bf16
+      // scales: 132 us with 4 steps, 113 with 8, 107 with 16, which loses where items are few: 32 experts of 768
+      // 372 against 345 us a block)
       g.tiles = (int)std::max<int64_t>(1, (8 * 128 + g.K - 1) / g.K);
       const int64_t all = (g.N + (GU ? 127 : 255)) / (GU ? 128 : 256), tiles = (all + g.tiles - 1) / g.tiles;
       const int64_t wgs = std::min<int64_t>(a.num_experts * tiles * g.sweeps, 1 << 16);

@@ -149,7 +149,7 @@ __device__ __forceinline__ void sumsq_wave_n(const float (&x)[NV][E], float (&ou
 // code = number of thresholds t_j (nthr <= 64 of them) with y >= fl(t_j * norm).  The thresholds come
 // from a register of the wave, one per lane, and the loop over them is the outer one: read from memory
 // inside the loop over elements, every comparison waited for a scalar load (8,192 vectors of 128 at
-// 4 bits, keys and values: 16.4 -> 9.9 us).
+// 4 bits, keys and values: 16.4 -> 9.9 us under the tracer).
 template <int NV, int E>
 __device__ __forceinline__ void count_thresholds_n(const float (&y)[NV][E], const float* __restrict__ thr, int nthr,
                                                    const float (&nrm)[NV], uint32_t (&code)[NV][E]) {

@@ -21,8 +21,8 @@
 // the two workgroups of a compute unit.  Few vectors (a decode step): one tile of 16, bound by one
 // compute unit's fetch of the two matrices and its matrix rate (2 x 2 vectors, D = 256: 27 us with
 // the caches flushed between calls, 45 us before the matrices were loaded whole; 8 x 2 vectors,
-// D = 128: 15 us).  TQ-MSE keys and values: transform and min/max arithmetic (8,192 vectors of 128
-// at 4 bits, keys and values: 9.3 us).  A step of 8 sequences (D = 128, 2 KV heads, 4 bits) was ~30
+// D = 128: 15 us; with the matrices in the L2 20 and 10).  TQ-MSE keys and values: transform and min/max arithmetic (8,192 vectors of 128
+// at 4 bits, keys and values: 8.1 us under the tracer, 6.6 back to back).  A step of 8 sequences (D = 128, 2 KV heads, 4 bits) was ~30
 // launches and 370 us before this kernel.
 #include <math.h>
 

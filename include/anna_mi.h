@@ -662,8 +662,8 @@ typedef struct {
   void* workspace;     /* anna_mi_moe_prefill_workspace bytes, 256-byte aligned */
   void* out;           /* [tokens][hidden_dim] */
 } anna_mi_moe_prefill_args;
-/* Bytes of workspace, or 0: not a call of this form (shape, too few routes per expert, or hidden rows
- * or weights that are not 16-byte aligned). */
+/* Bytes of workspace, or 0: not a call of this form (shape, hidden rows or weights that are not 16-byte
+ * aligned, or too few routes or too small a bank for it to be the faster one). */
 int64_t anna_mi_moe_prefill_workspace(const anna_mi_moe_prefill_args* args);
 int anna_mi_moe_prefill(const anna_mi_moe_prefill_args* args, void* stream);
 int64_t anna_mi_sizeof_moe_prefill_args(void);
