@@ -557,7 +557,9 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(const anna_
 constexpr int MERGE_DIM_WAVES = 4;
 constexpr int MERGE_DIM_MAXBLK = 64 * MERGE_DIM_WAVES;
 // PRE: partial values per lane loaded before the reductions -- a wave's whole share, 32 up to 128
-// blocks and 64 above (254 blocks with 32: 18.7 us, the rest of the share read in rounds of 8).
+// blocks, 48 up to 192 and 64 above.  With 32 and the rest of the share read in rounds of 8, 254 blocks took 18.7 us;
+// with 64 also for the fewer blocks, 130 to 160 of them took 0.8 us longer than that (one sequence of 8000
+// tokens, head_dim 128, one KV head: a decode of 14.2 us with 32, 15.4 with 64, 14.3 with 48).
 template <int MERGE_DIM_PRE>
 __global__ __launch_bounds__(64 * MERGE_DIM_WAVES) void decode_merge_dims_kernel(const anna_mi_decode_args a,
                                                                                  int64_t nblk) {
@@ -1576,6 +1578,8 @@ static int gqa_decode_splitkv_impl(const anna_mi_decode_args& a, void* stream) {
     const dim3 grid((unsigned)(a.head_dim / 64), (unsigned)a.q_heads, (unsigned)a.batch);
     if (nmerge <= 32 * MERGE_DIM_WAVES)
       hipLaunchKernelGGL(decode_merge_dims_kernel<32>, grid, dim3(64 * MERGE_DIM_WAVES), 0, st, a, nmerge);
+    else if (nmerge <= 48 * MERGE_DIM_WAVES)
+      hipLaunchKernelGGL(decode_merge_dims_kernel<48>, grid, dim3(64 * MERGE_DIM_WAVES), 0, st, a, nmerge);
     else
       hipLaunchKernelGGL(decode_merge_dims_kernel<64>, grid, dim3(64 * MERGE_DIM_WAVES), 0, st, a, nmerge);
     ANNA_LAUNCH_CHECK("decode_merge_dims_kernel");

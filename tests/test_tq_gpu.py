@@ -375,3 +375,16 @@ def test_splitkv_more_blocks_than_one_merge_workgroup(gpu, value_kind):
                                        32)[None]
         ref = _oracle_attention(f32(q), f32(k), vv, d ** -0.5)
         assert rel_err(f32(out), ref) <= BF16_TOL, qlen
+
+
+@pytest.mark.parametrize("blocks", [127, 128, 129, 191, 192, 193, 255, 256])
+def test_splitkv_merge_block_counts(gpu, blocks):
+    """The one-pass merge at both ends of what each of its instances holds ahead (fp32: blocks of exactly
+    16 tokens, the last one of 3)."""
+    torch.manual_seed(blocks)
+    n = 16 * (blocks - 1) + 3
+    q = torch.randn(2, 4, 1, 64, device=gpu)
+    k, v = (torch.randn(2, 2, n, 64, device=gpu) for _ in range(2))
+    out = torch.ops.anna.gqa_decode_splitkv_fused(q, k, v, 0.125, 16)
+    ref = _oracle_attention(f32(q), f32(k), f32(v), 0.125)
+    assert rel_err(f32(out), ref) <= 1e-5  # fp32 sums of 4096 terms at the most
