@@ -1013,17 +1013,32 @@ int launch_head_mfma(const void* x, int64_t M, int64_t K, int64_t xs, const uint
 
 // Where the dot2 forms stay faster for a few rows of x.  They give a workgroup 16 rows of W and a row of x its
 // own pass of products; the MFMA form gives a workgroup 64 and computes up to 16 rows of x at the price of one,
-// in passes of 16 128-k blocks per workgroup, whole ones also where K leaves some of a pass idle.  us, dot2 and
-// MFMA (bf16): K = 512 (12 of 16 blocks idle) M = 1, N = 1000 3.4 and 5.6, M = 4, N = 4096 4.8 and 5.9, M = 2,
-// N = 24576 7.0 and 8.0, but M = 4, N = 12288 6.4 and 6.0; K = 2048 M = 1, N = 4096 4.4 and 6.2, M = 2 5.4 and
-// 6.3, but M = 3 6.5 and 6.4; K = 4096 M = 1, N = 24576 14.0 and 15.6, M = 3, N = 1000 8.8 and 9.2, but M = 2,
-// N = 12288 12.5 and 10.8;
-// K = 8192 M = 1, N = 8192 15.8 and 17.2, but N = 12288 20.1 and 17.3.
+// in passes of 16 128-k blocks per workgroup, whole ones also where K leaves some of a pass idle.  So it depends on
+// how full the passes are, and for small grids on their rows.  us, dot2 and MFMA (bf16):
+//  - one row, passes less than 0.8 full: K = 512, N = 50000 8.8 and 14.1, N = 262144 34.6 and 47; K = 1024,
+//    N = 50000 10.7 and 14.0; K = 3072, N = 100000 40.0 and 46; but K = 2048, N = 50000 0.99 of the dot2 time, K = 4096,
+//    N = 151936 0.89, and past K = 4096, where the dot2 forms read x from memory, 0.6 to 0.9 from N = 16384 on;
+//  - a few rows, less than 0.7 full: K = 512, M = 2, N = 50000 11.4 and 14.1, M = 4, N = 8192 5.5 and 6.8; K = 1024,
+//    M = 2, N = 24576 1.12 of the dot2 time, N = 32768 0.95, M = 3, N = 8192 1.17, N = 12288 0.96;
+//  - else: K = 2048, M = 2, N = 8192 1.15, M = 3, N = 8192 0.95; K = 4096, M = 3, N = 4096 1.14, N = 8192 0.89;
+//    K = 3584, M = 4, N = 2000 1.17, K = 2048 0.90.
+// 1652 shapes (M 1 to 8, K 128 to 8192, N 1000 to 262144): 0.1% from the better form on average.
 bool tiled_dot2_faster(int64_t M, int64_t N, int64_t K) {
-  const int64_t blocks = K / 128, idle = (blocks + 15) / 16 * 16 - blocks;
-  if (K > 4096) return M <= 2 && M * M * N <= 8192;
-  if (K >= 512 && idle >= 8) return M <= (idle >= 12 ? 5 : 4) && N <= 32768 && M * M * N <= 98304;
-  return M <= (K < 512 ? 4 : K > 2048 ? 3 : 2) && M * M * N <= 24576;
+  const int64_t blocks = K / 128, passes = (blocks + 15) / 16 * 16;
+  const bool loose = 10 * blocks < 8 * passes, looser = 10 * blocks < 7 * passes;
+  if (M == 1) return (loose && K > 128 && K <= 4096) || N <= (K <= 4096 ? 24576 : 12288);
+  if (looser && K > 128 && K <= 4096) return K > 256 && K <= 512 ? M <= 6 && M * M * N <= 221184 : M <= 5 && M * M * N <= 98304;
+  return M <= (loose || K > 2048 ? 4 : 3) && M * N <= (loose ? 24576 : 16384);
+}
+
+// Where the dot2 GEMV and the chunk lists stay faster than the MFMA form with the selection over its blocks (which
+// reads less, and takes any k): few k and one row, where the GEMV's lead is more than the selection saves (K = 512,
+// V = 262144 50.5 and 59.8 us; K = 2560, V = 151936 1.28 of the steps' time, V = 32768 1.01), and short vocabularies of
+// a long K (K = 2560, V = 8192, one and two rows 1.12 and 1.10; V = 12288 1.04 and 0.95).
+bool head_steps_faster(int64_t rows, int64_t V, int64_t K, int64_t k) {
+  if (k > 8 || rows > 2 || !tiled_dot2_faster(rows, V, K)) return false;
+  if (K > 2304 && V < 12288) return true;
+  return rows == 1 && V >= 50000 && ((K > 256 && K <= 512) || K > 2304);
 }
 
 // ANNA_MI_TILED_PLAIN=1 keeps the tiled GEMV off its LDS-staged form (for comparisons and tests)
@@ -1201,7 +1216,7 @@ extern "C" int anna_mi_lm_head_int4_topk_ws(const void* x, int x_dtype, int64_t 
     fused = head_mfma_ok<XDT>(x, rows, K, x_row_stride, qweight, tile, group_size) && !g_tiled_plain;
   });
   // (short rows: one workgroup reads them whole)
-  if (!fused || C > TKB_MAX_BLOCKS || vocab < 8192 || vocab >= INT32_MAX || top_k < 1 || top_k > TK_MAX)
+  if (!fused || head_steps_faster(rows, vocab, K, top_k) || C > TKB_MAX_BLOCKS || vocab < 8192 || vocab >= INT32_MAX || top_k < 1 || top_k > TK_MAX)
     return anna_mi_lm_head_int4_topk(x, x_dtype, rows, K, x_row_stride, qweight, tiles, packed_cols, tile, qscale,
                                      scale_dtype, qzeros, group_count, scale_stride_group, scale_stride_row, group_size,
                                      vocab, top_k, workspace, values, indices, stream);

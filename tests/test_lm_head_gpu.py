@@ -150,10 +150,13 @@ def test_lm_head_topk_exact_ties_in_wave_path(gpu, layout):
     (128, 8192, 1, 1, torch.bfloat16, 128), (256, 8196, 2, 8, torch.float16, 128), (512, 9000, 3, 32, torch.bfloat16, 128),
     (640, 16444, 5, 20, torch.float16, 128), (1024, 70004, 9, 8, torch.bfloat16, 256),
     (2048, 12300, 17, 9, torch.bfloat16, 128), (2176, 8260, 33, 5, torch.float16, 128),
+    (512, 49996, 1, 8, torch.bfloat16, 128), (512, 50000, 1, 8, torch.bfloat16, 128), (512, 50000, 1, 9, torch.float16, 128),
+    (2560, 50000, 1, 3, torch.float16, 128), (2432, 12284, 2, 3, torch.float16, 128), (2432, 12288, 2, 3, torch.bfloat16, 128),
 ])
 def test_lm_head_block_selection(gpu, k, n, rows, top_k, dtype, group):
     """Whole 128-k blocks on tiles of 4 rows: the MFMA GEMV (K short of four waves' shares, ragged last
-    block of rows, one to three 16-row blocks of x) and the selection over 64-logit blocks, against fp64;
+    block of rows, one to three 16-row blocks of x) and the selection over 64-logit blocks, and the shapes that
+    take the GEMV and the chunk lists instead, against fp64;
     repeated weight rows make exact ties, which go to the lower index."""
     torch.manual_seed(k + n)
     kp = -(-k // group) * group
@@ -190,7 +193,11 @@ def test_lm_head_block_selection(gpu, k, n, rows, top_k, dtype, group):
 @pytest.mark.parametrize("m,n,k", [(1, 24576, 128), (1, 24580, 128), (4, 1536, 256), (4, 1540, 256), (5, 300, 256),
                                    (5, 3932, 512), (5, 3936, 512), (1, 32768, 512), (1, 32772, 512), (6, 300, 512),
                                    (4, 6144, 768), (4, 6148, 768), (5, 300, 768), (2, 6144, 1152), (2, 6148, 1536),
-                                   (3, 300, 2048), (3, 2728, 4096), (3, 2732, 4096), (2, 2048, 4224), (2, 2052, 4224), (3, 300, 4224)])
+                                   (3, 300, 2048), (3, 2728, 4096), (3, 2732, 4096), (2, 2048, 4224), (2, 2052, 4224), (3, 300, 4224),
+                                   (6, 6144, 512), (6, 6148, 512), (2, 55296, 384), (2, 55300, 384), (5, 3936, 768),
+                                   (6, 300, 768), (4, 6144, 1536), (4, 6148, 1536), (1, 50000, 1536), (3, 5460, 2048),
+                                   (3, 5464, 2048), (4, 300, 2048), (4, 4096, 2176), (4, 4096, 4096), (4, 4100, 4096), (1, 24580, 2048), (4, 6144, 4224), (4, 6148, 4224),
+                                   (1, 12288, 4224), (1, 12292, 4224)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_tiled_gemv_on_both_sides_of_its_forms(gpu, m, n, k, dtype):
     """Tiles of 4 rows and whole 128-k blocks: the dot2 forms for few rows, the MFMA form beyond."""
